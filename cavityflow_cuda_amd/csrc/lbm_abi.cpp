@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cfloat>
 #include <cmath>
 #include <cstdio>
@@ -149,6 +150,38 @@ int copy_set(lbm_solver* s, int field, const Box& b, int ncomp, const void* src,
     LBM_HIP(launch_box_set(s, field, b, s->staging, mask, st), "box set kernel");
     LBM_HIP(hipStreamSynchronize(st), "hipStreamSynchronize");
     return LBM_OK;
+}
+
+// Bytes of domains stepped so far on each device (modulo the array): how much
+// passed between two half-steps of one solver says whether its state can still
+// be in the caches. Only launch shapes depend on it, never results.
+std::atomic<uint64_t> g_stepped[64];
+
+// The launch options of a step: the ones set (or the defaults by face work and
+// size), and for whole-domain steps without face work of a kernel the caller
+// has not set, step_options for the bytes stepped between this solver's
+// half-steps.
+int options_of_step(lbm_solver* s, int kernel, const Box& b)
+{
+    const bool full = is_full(s, b);
+    const uint64_t bytes = resident_bytes(s) / (uint64_t)s->n * b.cells();
+    const uint64_t now = g_stepped[s->p.device & 63].fetch_add(bytes, std::memory_order_relaxed);
+    // relaxed atomics: threads that step boxes of one solver side by side may
+    // both write the marks
+    const int last = __atomic_exchange_n(&s->last_kernel, kernel, __ATOMIC_RELAXED);
+    uint64_t gap = __atomic_load_n(&s->step_gap[0], __ATOMIC_RELAXED);
+    uint64_t gap_before = __atomic_load_n(&s->step_gap[1], __ATOMIC_RELAXED);
+    if (full || kernel != last) {   // box steps of one half-step share its mark
+        gap_before = gap;
+        gap = last < 0 ? 0 : now - __atomic_load_n(&s->step_mark, __ATOMIC_RELAXED);
+        __atomic_store_n(&s->step_gap[1], gap_before, __ATOMIC_RELAXED);
+        __atomic_store_n(&s->step_gap[0], gap, __ATOMIC_RELAXED);
+        __atomic_store_n(&s->step_mark, now, __ATOMIC_RELAXED);
+    }
+    if (!full || s->launch_set[kernel] || s->xpack[0] || s->xpack[1] || s->xunpack[0] ||
+        s->xunpack[1] || !plane_off32(s))
+        return s->launch[kernel];
+    return step_options(s, kernel, std::min(gap, gap_before), std::max(gap, gap_before));
 }
 
 // norm . c_l > 0 mask of setDensityDistributions(..., direction, ...)
@@ -377,6 +410,7 @@ int lbm_create(const lbm_params* params, lbm_solver** out)
     s->launch[0] = default_launch(p.precision, 0, false, s->n >= kWideCells);
     s->launch[1] = default_launch(p.precision, 1, false, s->n >= kWideCells);
     s->launch_set[0] = s->launch_set[1] = 0;
+    s->last_kernel = -1;
     // round inv_tau / lid / gravity to the arithmetic type once
     if (p.precision != LBM_F64) {
         s->p.inv_tau = (float)p.inv_tau;
@@ -489,7 +523,7 @@ int lbm_simulation_step_alpha(lbm_solver* s, const int origin[3], const int size
         return rc;
     if ((rc = set_device(s)))
         return rc;
-    LBM_HIP(launch_alpha(s, b, stream), "alpha kernel launch");
+    LBM_HIP(launch_alpha(s, b, options_of_step(s, 0, b), stream), "alpha kernel launch");
     return LBM_OK;
 }
 
@@ -502,7 +536,7 @@ int lbm_simulation_step_beta(lbm_solver* s, const int origin[3], const int size[
         return rc;
     if ((rc = set_device(s)))
         return rc;
-    LBM_HIP(launch_beta(s, b, stream), "beta kernel launch");
+    LBM_HIP(launch_beta(s, b, options_of_step(s, 1, b), stream), "beta kernel launch");
     return LBM_OK;
 }
 

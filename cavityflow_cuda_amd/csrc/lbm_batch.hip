@@ -35,7 +35,8 @@ struct MemberDesc {
     int32_t n, nx, nxy;
     uint32_t tile_begin;
     int32_t store_rho, store_u;
-    double inv_tau, lid, g0, g1, g2;
+    double inv_tau, lid, g0, g1, g2, rest_rho;
+    int32_t gravity;
     uint32_t* status;
 };
 
@@ -56,6 +57,8 @@ __device__ __forceinline__ StepArgs<C> member_args(const MemberDesc& d, int phas
     a.g0 = (C)d.g0;
     a.g1 = (C)d.g1;
     a.g2 = (C)d.g2;
+    a.gravity = d.gravity;
+    a.rest_rho = (C)d.rest_rho;
     a.store_rho = d.store_rho;
     a.store_u = d.store_u;
     a.xpack_on = 0;
@@ -129,7 +132,7 @@ __global__ __launch_bounds__(BLOCK) void k_batch(const MemberDesc* __restrict__ 
                     continue;
                 if (wrap) {
                     // the wrap path addresses planes from the unshifted base
-                    const Acc64<S, true> acc{(S*)plane0, a.stride, (int32_t)id, a.n};
+                    const AccWrap32<S> acc{plane0, a.stride, (int32_t)id, a.n};
                     beta_cell<P, kXfNone>(a, id, ((const LBM_GLOBAL uint8_t*)a.flags)[id], acc);
                 } else {
                     const Acc32<S, false> acc{a.plane, id * (uint32_t)sizeof(S)};
@@ -357,6 +360,8 @@ int prepare_pairs(lbm_batch* b, int pairs)
         d.g0 = h.g0;
         d.g1 = h.g1;
         d.g2 = h.g2;
+        d.gravity = h.gravity;
+        d.rest_rho = h.rest_rho;
         d.status = s->status;
         map.insert(map.end(), (size_t)d.tiles_x * d.tiles_y * d.chunks, (int32_t)m);
     }
@@ -382,7 +387,8 @@ int prepare_pairs(lbm_batch* b, int pairs)
 int apply_tuning(lbm_batch* b, const lbm_batch_tuning& t)
 {
     if (t.block == 1024 && b->precision == LBM_F64) {
-        // 1024 threads leave 128 VGPRs per thread: the FP64 kernels would spill
+        // a limit from when the FP64 kernels needed more than the 128 VGPRs of
+        // such a workgroup's threads (87 and 71 now)
         set_error("batch tuning: FP64 members take workgroups of 256 or 512 threads");
         return LBM_ERR_UNSUPPORTED;
     }
@@ -613,6 +619,8 @@ int lbm_batch_create(lbm_solver* const* members, int count, lbm_batch** out)
         d.g0 = s->p.gravitation[0];
         d.g1 = s->p.gravitation[1];
         d.g2 = s->p.gravitation[2];
+        d.gravity = has_gravity(s->p.gravitation);
+        d.rest_rho = gravity_product(d.g0, d.g1, d.g2);
         d.status = s->status;
     }
     lbm_batch_tuning t;
@@ -816,8 +824,8 @@ int lbm_batch_autotune(lbm_batch* b, int trial_steps, hipStream_t stream,
         return LBM_OK;
     };
     const lbm_batch_tuning start = best;
-    // 1024-thread workgroups: not for FP64 (register spills), and at most two
-    // are resident per CU
+    // 1024-thread workgroups: not for FP64 (apply_tuning), and at most two are
+    // resident per CU
     const int max_block = b->precision == LBM_F64 ? 512 : 1024;
     for (int blk : {256, 512, 1024})
         for (int cpt : {1, 2, 4})

@@ -35,8 +35,14 @@ __device__ __forceinline__ uint32_t box_cell(const StepArgs<C>& a, uint32_t gid)
 // beta neighbour shift is folded into it) and one 32-bit byte offset per lane
 // shared by all 19 planes, so every access is a saddr global load/store with
 // no per-plane vector address arithmetic; it needs cells * sizeof(S) < 2^32.
-// Acc64 uses a 64-bit element index per plane and, with WRAP, the reference's
-// linear-index wrap (domainWrap, CLbmBetaCPU.cpp:44-50).
+// AccWrap32 serves the same planes where the reference's linear-index wrap
+// (domainWrap, CLbmBetaCPU.cpp:44-50) may apply: a uniform unshifted base and
+// a wrapped 32-bit offset per plane. Acc64 uses a 64-bit element index per
+// plane, with WRAP the wrap as well.
+// for_stores() gives the accessor a step's stores go through: a fresh (empty
+// asm) copy of the lane's offset or index, from which the addresses are formed
+// anew. Without it the compiler keeps the loads' addresses live across the
+// collision: 19 VGPR pairs, or 38 VGPRs of wrapped indices.
 // The plane bases come precomputed in the kernel arguments: opaque uniform
 // values the compiler cannot fold into per-lane pointer chains.
 // Every population array is device (global) memory. The accessors say so
@@ -45,10 +51,18 @@ __device__ __forceinline__ uint32_t box_cell(const StepArgs<C>& a, uint32_t gid)
 // instructions, which wait on both memory counters.
 #define LBM_GLOBAL __attribute__((address_space(1)))
 
+template <class T>
+__device__ __forceinline__ T fresh(T v)
+{
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
 template <class S, bool NT>
 struct Acc32 {
     const char* const* plane;
     uint32_t off;
+    __device__ __forceinline__ Acc32 for_stores() const { return {plane, fresh(off)}; }
     __device__ __forceinline__ S load(int l, int32_t) const
     {
         const LBM_GLOBAL S* p = (const LBM_GLOBAL S*)(plane[l] + off);
@@ -58,17 +72,37 @@ struct Acc32 {
     }
     __device__ __forceinline__ void store(int l, int32_t, S v) const
     {
-        // A fresh copy of the offset keeps the compiler from reusing the
-        // loads' 64-bit addresses (19 VGPR pairs kept live across the
-        // collision): each store then takes the uniform base + 32-bit offset
-        // form, as the loads do.
-        uint32_t o = off;
-        asm volatile("" : "+v"(o));
-        LBM_GLOBAL S* p = (LBM_GLOBAL S*)(const_cast<char*>(plane[l]) + o);
+        LBM_GLOBAL S* p = (LBM_GLOBAL S*)(const_cast<char*>(plane[l]) + off);
         if (NT)
             __builtin_nontemporal_store(v, p);
         else
             *p = v;
+    }
+};
+
+// id + delta wrapped into [0, n) once, as the reference does.
+__device__ __forceinline__ int32_t wrapped(int32_t id, int32_t delta, int32_t n)
+{
+    int32_t j = id + delta;
+    j = (j >= n) ? j - n : j;
+    return (j < 0) ? j + n : j;
+}
+
+template <class S>
+struct AccWrap32 {
+    const char* dd;
+    int64_t stride;
+    int32_t id, n;
+    __device__ __forceinline__ AccWrap32 for_stores() const { return {dd, stride, fresh(id), n}; }
+    __device__ __forceinline__ S load(int l, int32_t delta) const
+    {
+        const char* base = dd + (int64_t)l * stride * (int64_t)sizeof(S);
+        return *(const LBM_GLOBAL S*)(base + (uint32_t)wrapped(id, delta, n) * (uint32_t)sizeof(S));
+    }
+    __device__ __forceinline__ void store(int l, int32_t delta, S v) const
+    {
+        char* base = const_cast<char*>(dd) + (int64_t)l * stride * (int64_t)sizeof(S);
+        *(LBM_GLOBAL S*)(base + (uint32_t)wrapped(id, delta, n) * (uint32_t)sizeof(S)) = v;
     }
 };
 
@@ -77,14 +111,10 @@ struct Acc64 {
     S* dd;
     int64_t stride;
     int32_t id, n;
+    __device__ __forceinline__ Acc64 for_stores() const { return {dd, stride, fresh(id), n}; }
     __device__ __forceinline__ int64_t index(int l, int32_t delta) const
     {
-        int32_t j = id + delta;
-        if (WRAP) {
-            j = (j >= n) ? j - n : j;
-            j = (j < 0) ? j + n : j;
-        }
-        return (int64_t)l * stride + j;
+        return (int64_t)l * stride + (WRAP ? wrapped(id, delta, n) : id + delta);
     }
     __device__ __forceinline__ S load(int l, int32_t delta) const
     {
@@ -215,12 +245,119 @@ __device__ __forceinline__ typename P::C xunpack_value(typename P::C r, int l, u
     return P::load(P::store_checked(r, l, ov), l);
 }
 
+// -------------------------------------------------------------- collision ---
+
+// Both directions of an opposite pair with velocity +-v and weight w, the
+// equilibria of common.h:132-160: w * (rho + (+-3 v) + 4.5 v^2). -3 v is
+// exactly -(3 v), so the pair shares 3 v and 4.5 v^2 with every result's bits
+// kept; with the 16-bit formats and with domains that stay in the Infinity
+// Cache the steps are as much bound by instructions as by memory.
+template <class C>
+__device__ __forceinline__ void equilibrium_pair(C& fp, C& fm, C rho, C v, C w)
+{
+    const C t = (C)3 * v, q = ((C)9 / (C)2) * (v * v);
+    fp = w * ((rho + t) + q);
+    fm = w * ((rho - t) + q);
+}
+
+// Applies op(direction, opposite, velocity, weight) to the nine opposite pairs,
+// one after the other: few values live beside the 19 populations.
+template <class C, class Op>
+__device__ __forceinline__ void for_pairs(C ux, C uy, C uz, Op op)
+{
+    constexpr C wa = (C)1 / (C)18, wd = (C)1 / (C)36;
+    op(0, 1, ux, wa);
+    op(2, 3, uy, wa);
+    op(4, 5, ux + uy, wd);
+    op(6, 7, ux - uy, wd);
+    op(8, 9, ux + uz, wd);
+    op(10, 11, ux - uz, wd);
+    op(12, 13, uy + uz, wd);
+    op(14, 15, uy - uz, wd);
+    op(16, 17, uz, wa);
+}
+
+// d += inv_tau * (eq - d) in every direction; terms(l) may add to each opposite
+// pair (l, l + 1), and put(l) stores direction l. rho is the reference's
+// dd_param. 4- and 8-byte populations are stored as soon as their pair has its
+// values: the stores spread over the collision (62^3 FP32 13.5 us a pair of
+// steps against 13.8 with all stores at the end, 229 x 186 x 141 with outputs
+// 354 against 359). 2-byte ones all at the end (LATE; 512^3 F16S 3.74 ms
+// against 3.81): the empty statements that read the results keep the stores
+// behind them.
+template <bool LATE, class C, class Terms, class Put>
+__device__ __forceinline__ void relax(C (&d)[kQ], C rho, C ux, C uy, C uz, C inv_tau, Terms terms,
+                                      Put put)
+{
+    for_pairs(ux, uy, uz, [&](int p, int m, C v, C w) {
+        C ep, em;
+        equilibrium_pair(ep, em, rho, v, w);
+        d[p] += inv_tau * (ep - d[p]);
+        d[m] += inv_tau * (em - d[m]);
+        terms(p);
+        if (!LATE) {
+            put(p);
+            put(m);
+        }
+    });
+    d[18] += inv_tau * (eq_18(rho) - d[18]);
+    if (!LATE) {
+        put(18);
+        return;
+    }
+#pragma unroll
+    for (int l = 0; l < kQ; l++)
+        d[l] = fresh(d[l]);
+#pragma unroll
+    for (int l = 0; l < kQ; l++)
+        put(l);
+}
+
+// A VELOCITY_INJECTION cell takes the equilibrium of the lid velocity and
+// rho = 1 instead of relaxing: with d = 0 and inv_tau = 1 the relaxation gives
+// 0 + 1 * (eq - 0), the equilibrium's own bits. The test is on the whole wave:
+// waves without a lid cell pay one scalar branch, not 19 selects or copies.
+template <class C>
+__device__ __forceinline__ void inject(bool lid_cell, C (&d)[kQ], C& rho, C& ux, C& uy, C& uz,
+                                       C& inv_tau, C lid)
+{
+    if (!__builtin_amdgcn_ballot_w64(lid_cell))
+        return;
+#pragma unroll
+    for (int l = 0; l < kQ; l++)
+        d[l] = lid_cell ? (C)0 : d[l];
+    inv_tau = lid_cell ? (C)1 : inv_tau;
+    ux = lid_cell ? lid : ux;
+    uy = lid_cell ? (C)0 : uy;
+    uz = lid_cell ? (C)0 : uz;
+    rho = lid_cell ? (C)1 : rho;
+}
+
+// The gravity terms of alpha (CLbmAlphaCPU.cpp:199-325): the k-th scales the
+// one before it (the reference's `tmp` is a #define for `rho`, the first
+// scales rho itself), and is added to direction 2 k and subtracted from
+// 2 k + 1.
+template <class C>
+__device__ __forceinline__ C gravity_factor(int k, C g0, C g1, C g2)
+{
+    switch (k) {
+    case 0: return g0 * ((C)1 / (C)18);
+    case 1: return g1 * ((C)-1 / (C)18);
+    case 2: return (g0 - g1) * ((C)1 / (C)36);
+    case 3: return (g0 + g1) * ((C)1 / (C)36);
+    case 4: return (g0 + g2) * ((C)1 / (C)36);
+    case 5: return (g0 - g2) * ((C)1 / (C)36);
+    case 6: return (g2 - g1) * ((C)1 / (C)36);
+    case 7: return (g2 + g1) * ((C)-1 / (C)36);
+    default: return g2 * ((C)1 / (C)18);
+    }
+}
+
 // ----------------------------------------------------------------- alpha ---
 
 // One cell of CLbmAlphaCPU::alphaKernelCPU (CLbmAlphaCPU.cpp:75-494). The
-// reference's `tmp` is a #define for `rho` (:199): every gravity term
-// overwrites rho and the stored density is the last gravity term. `flag` is
-// the cell's flag, passed in so a caller that already holds it skips a load.
+// stored density is the last gravity term (add_gravity). `flag` is the cell's
+// flag, passed in so a caller that already holds it skips a load.
 template <class P, int XF = kXfPack, class A>
 __device__ __forceinline__ void alpha_cell(const StepArgs<typename P::C>& a, uint32_t id,
                                            int flag, const A& acc)
@@ -279,104 +416,35 @@ __device__ __forceinline__ void alpha_cell(const StepArgs<typename P::C>& a, uin
     moments(d, rho, ux, uy, uz);
 
     if (flag == kFluid || flag == kVelocityInjection) {
-        const C inv_tau = a.inv_tau;
-        const C g0 = a.g0, g1 = a.g1, g2 = a.g2;
-        const bool fluid = (flag == kFluid);
-        C vel2, vela2, vab, dd_param;
-        C e[kQ];
-        if (!fluid) {
-            ux = a.lid;
-            uy = (C)0;
-            uz = (C)0;
-            rho = (C)1;
-        }
-        vel2 = ux * ux + uy * uy + uz * uz;
-        dd_param = rho - ((C)3 / (C)2) * vel2;
-        // post-collision value of direction l: relaxation for FLUID (d += inv_tau*(eq - d)),
-        // the equilibrium itself for VELOCITY_INJECTION
-#define LBM_RELAX(l, eqv) e[l] = fluid ? (d[l] + inv_tau * ((eqv) - d[l])) : (eqv)
-        rho = g0 * ((C)1 / (C)18) * rho;
-        vela2 = ux * ux;
-        LBM_RELAX(1, eq_a1(ux, vela2, dd_param));
-        e[1] -= rho;
-        LBM_RELAX(0, eq_a0(ux, vela2, dd_param));
-        e[0] += rho;
-
-        rho = g1 * ((C)-1 / (C)18) * rho;
-        vela2 = uy * uy;
-        LBM_RELAX(3, eq_a1(uy, vela2, dd_param));
-        e[3] -= rho;
-        LBM_RELAX(2, eq_a0(uy, vela2, dd_param));
-        e[2] += rho;
-
-        vab = ux + uy;
-        vela2 = vab * vab;
-        rho = (g0 - g1) * ((C)1 / (C)36) * rho;
-        LBM_RELAX(5, eq_5(vab, vela2, dd_param));
-        e[5] -= rho;
-        LBM_RELAX(4, eq_4(vab, vela2, dd_param));
-        e[4] += rho;
-
-        vab = ux - uy;
-        vela2 = vab * vab;
-        rho = (g0 + g1) * ((C)1 / (C)36) * rho;
-        LBM_RELAX(7, eq_5(vab, vela2, dd_param));
-        e[7] -= rho;
-        LBM_RELAX(6, eq_4(vab, vela2, dd_param));
-        e[6] += rho;
-
-        vab = ux + uz;
-        vela2 = vab * vab;
-        rho = (g0 + g2) * ((C)1 / (C)36) * rho;
-        LBM_RELAX(9, eq_5(vab, vela2, dd_param));
-        e[9] -= rho;
-        LBM_RELAX(8, eq_4(vab, vela2, dd_param));
-        e[8] += rho;
-
-        rho = (g0 - g2) * ((C)1 / (C)36) * rho;
-        vab = ux - uz;
-        vela2 = vab * vab;
-        LBM_RELAX(11, eq_5(vab, vela2, dd_param));
-        e[11] -= rho;
-        LBM_RELAX(10, eq_4(vab, vela2, dd_param));
-        e[10] += rho;
-
-        vab = uy + uz;
-        vela2 = vab * vab;
-        rho = (g2 - g1) * ((C)1 / (C)36) * rho;
-        LBM_RELAX(13, eq_5(vab, vela2, dd_param));
-        e[13] -= rho;
-        LBM_RELAX(12, eq_4(vab, vela2, dd_param));
-        e[12] += rho;
-
-        vab = uy - uz;
-        vela2 = vab * vab;
-        rho = (g2 + g1) * ((C)-1 / (C)36) * rho;
-        LBM_RELAX(15, eq_5(vab, vela2, dd_param));
-        e[15] -= rho;
-        LBM_RELAX(14, eq_4(vab, vela2, dd_param));
-        e[14] += rho;
-
-        vela2 = uz * uz;
-        rho = g2 * ((C)1 / (C)18) * rho;
-        LBM_RELAX(17, eq_a1(uz, vela2, dd_param));
-        e[17] -= rho;
-        LBM_RELAX(16, eq_a0(uz, vela2, dd_param));
-        e[16] += rho;
-
-        LBM_RELAX(18, eq_18(dd_param));
-#undef LBM_RELAX
+        C inv_tau = a.inv_tau;
+        inject(flag == kVelocityInjection, d, rho, ux, uy, uz, inv_tau, a.lid);
+        const C vel2 = ux * ux + uy * uy + uz * uz;
         // direction l goes to slot opp(l) of this cell
         uint32_t ov = 0;
-#pragma unroll
-        for (int l = 0; l < kQ; l++)
-            acc.store(opp(l), 0, P::store_checked(e[l], opp(l), ov));
+        const A to = acc.for_stores();
+        // Without gravity its terms add +-0 to every direction, which changes
+        // nothing as long as rho is finite, and leave +-0 as the stored density
+        // (rest_rho * rho has its sign); a non-finite rho makes every term NaN,
+        // so waves that hold one take them too.
+        const bool terms = a.gravity || __builtin_amdgcn_ballot_w64(!__builtin_isfinite(rho));
+        C term = rho;
+        relax<sizeof(typename P::S) == 2>(
+            d, rho - ((C)3 / (C)2) * vel2, ux, uy, uz, inv_tau,
+            [&](int l) {
+                if (terms) {
+                    term = gravity_factor(l / 2, a.g0, a.g1, a.g2) * term;
+                    d[l + 1] -= term;
+                    d[l] += term;
+                }
+            },
+            [&](int l) { to.store(opp(l), 0, P::store_checked(d[l], opp(l), ov)); });
+        rho = terms ? term : a.rest_rho * rho;
         raise_overflow<P>(a.status, ov);
         if (pack) {
             C out[kQ];
 #pragma unroll
             for (int s2 = 0; s2 < kQ; s2++)
-                out[s2] = e[opp(s2)];
+                out[s2] = d[opp(s2)];
             xpack_alpha<P>(a, row, pl, pr, out);
         }
     } else if (flag == kObstacle) {
@@ -460,86 +528,20 @@ __device__ __forceinline__ void beta_cell(const StepArgs<typename P::C>& a, uint
     C rho, ux, uy, uz;
     moments(d, rho, ux, uy, uz);
 
-    if (flag == kFluid) {
-        const C inv_tau = a.inv_tau;
-        C vel2 = ux * ux + uy * uy + uz * uz;
-        rho = rho - ((C)3 / (C)2) * (vel2);
-        C vela2 = ux * ux;
-        d[0] += inv_tau * (eq_a0(ux, vela2, rho) - d[0]);
-        d[1] += inv_tau * (eq_a1(ux, vela2, rho) - d[1]);
-        vela2 = uy * uy;
-        d[2] += inv_tau * (eq_a0(uy, vela2, rho) - d[2]);
-        d[3] += inv_tau * (eq_a1(uy, vela2, rho) - d[3]);
-        vel2 = ux + uy;
-        vela2 = vel2 * vel2;
-        d[4] += inv_tau * (eq_4(vel2, vela2, rho) - d[4]);
-        d[5] += inv_tau * (eq_5(vel2, vela2, rho) - d[5]);
-        vel2 = ux - uy;
-        vela2 = vel2 * vel2;
-        d[6] += inv_tau * (eq_4(vel2, vela2, rho) - d[6]);
-        d[7] += inv_tau * (eq_5(vel2, vela2, rho) - d[7]);
-        vel2 = ux + uz;
-        vela2 = vel2 * vel2;
-        d[8] += inv_tau * (eq_4(vel2, vela2, rho) - d[8]);
-        d[9] += inv_tau * (eq_5(vel2, vela2, rho) - d[9]);
-        vel2 = ux - uz;
-        vela2 = vel2 * vel2;
-        d[10] += inv_tau * (eq_4(vel2, vela2, rho) - d[10]);
-        d[11] += inv_tau * (eq_5(vel2, vela2, rho) - d[11]);
-        vel2 = uy + uz;
-        vela2 = vel2 * vel2;
-        d[12] += inv_tau * (eq_4(vel2, vela2, rho) - d[12]);
-        d[13] += inv_tau * (eq_5(vel2, vela2, rho) - d[13]);
-        vel2 = uy - uz;
-        vela2 = vel2 * vel2;
-        d[14] += inv_tau * (eq_4(vel2, vela2, rho) - d[14]);
-        d[15] += inv_tau * (eq_5(vel2, vela2, rho) - d[15]);
-        vela2 = uz * uz;
-        d[16] += inv_tau * (eq_a0(uz, vela2, rho) - d[16]);
-        d[17] += inv_tau * (eq_a1(uz, vela2, rho) - d[17]);
-        d[18] += inv_tau * (eq_18(rho) - d[18]);
-    } else if (flag == kVelocityInjection) {
-        ux = a.lid;
-        uy = (C)0;
-        uz = (C)0;
-        rho = (C)1;
-        C vel2 = ux * ux + uy * uy + uz * uz;
-        rho = rho - ((C)3 / (C)2) * vel2;
-        C vela2 = ux * ux;
-        d[0] = eq_a0(ux, vela2, rho);
-        d[1] = eq_a1(ux, vela2, rho);
-        vela2 = uy * uy;
-        d[2] = eq_a0(uy, vela2, rho);
-        d[3] = eq_a1(uy, vela2, rho);
-        vel2 = ux + uy;
-        vela2 = vel2 * vel2;
-        d[4] = eq_4(vel2, vela2, rho);
-        d[5] = eq_5(vel2, vela2, rho);
-        vel2 = ux - uy;
-        vela2 = vel2 * vel2;
-        d[6] = eq_4(vel2, vela2, rho);
-        d[7] = eq_5(vel2, vela2, rho);
-        vel2 = ux + uz;
-        vela2 = vel2 * vel2;
-        d[8] = eq_4(vel2, vela2, rho);
-        d[9] = eq_5(vel2, vela2, rho);
-        vel2 = ux - uz;
-        vela2 = vel2 * vel2;
-        d[10] = eq_4(vel2, vela2, rho);
-        d[11] = eq_5(vel2, vela2, rho);
-        vel2 = uy + uz;
-        vela2 = vel2 * vel2;
-        d[12] = eq_4(vel2, vela2, rho);
-        d[13] = eq_5(vel2, vela2, rho);
-        vel2 = uy - uz;
-        vela2 = vel2 * vel2;
-        d[14] = eq_4(vel2, vela2, rho);
-        d[15] = eq_5(vel2, vela2, rho);
-        vela2 = uz * uz;
-        d[16] = eq_a0(uz, vela2, rho);
-        d[17] = eq_a1(uz, vela2, rho);
-        d[18] = eq_18(rho);
-    } else if (flag == kObstacle) {
+    // direction l goes to slot l of neighbour id + c_l
+    uint32_t ov = 0;
+    auto put = [&](const A& to, int l) {
+        to.store(l, cx(l) + cy(l) * a.nx + cz(l) * a.nxy, P::store_checked(d[l], l, ov));
+    };
+    // The collision comes last: a branch after it that still read the arriving
+    // values would keep all 19 in registers of their own (FP32 64 VGPRs instead
+    // of 40, FP64 118 instead of 70). `kind` goes through an empty statement so
+    // that the branches stay in this order.
+    constexpr int kStill = 0, kPass = 1, kMoving = 2;
+    const int kind = fresh(flag == kFluid || flag == kVelocityInjection ? kMoving
+                           : flag == kObstacle                          ? kStill
+                                                                        : kPass);
+    if (kind == kStill) {
         if (pack) {
             // the swap writes back the value read from plane l (:302-311)
             C out[kQ];
@@ -554,17 +556,24 @@ __device__ __forceinline__ void beta_cell(const StepArgs<typename P::C>& a, uint
             uz = (C)0;
         }
     }
-
-    if (flag != kObstacle) {
-        // direction l goes to slot l of neighbour id + c_l
-        uint32_t ov = 0;
+    if (kind == kPass) {
+        const A to = acc.for_stores();
 #pragma unroll
         for (int l = 0; l < kQ; l++)
-            acc.store(l, cx(l) + cy(l) * a.nx + cz(l) * a.nxy, P::store_checked(d[l], l, ov));
-        raise_overflow<P>(a.status, ov);
-        if (pack)
-            xpack_beta<P>(a, row, pl, pr, d);
+            put(to, l);
     }
+    if (kind == kMoving) {
+        C inv_tau = a.inv_tau;
+        inject(flag == kVelocityInjection, d, rho, ux, uy, uz, inv_tau, a.lid);
+        const C vel2 = ux * ux + uy * uy + uz * uz;
+        rho = rho - ((C)3 / (C)2) * (vel2);
+        const A to = acc.for_stores();
+        relax<sizeof(typename P::S) == 2>(d, rho, ux, uy, uz, inv_tau, [](int) {},
+                                          [&](int l) { put(to, l); });
+    }
+    raise_overflow<P>(a.status, ov);
+    if (pack && kind != kStill)
+        xpack_beta<P>(a, row, pl, pr, d);
 
     if (a.store_u) {
         a.u[id] = ux;

@@ -54,6 +54,8 @@ struct StepArgs {
     uint32_t cells;   // cells of the box
     FastDiv div_bx, div_by;
     C inv_tau, lid, g0, g1, g2;
+    int gravity;      // any of g0, g1, g2 is not zero
+    C rest_rho;       // gravity_product, used when g is zero
     int store_rho, store_u;
     int xcd;          // renumber workgroups per XCD
     // byte address of plane l, shifted by the neighbour offset of direction l
@@ -70,6 +72,17 @@ struct StepArgs {
     // set to 1 by a store the storage format cannot represent (F16C)
     uint32_t* status;
 };
+
+// What alpha's gravity terms multiply rho by in all (CLbmAlphaCPU.cpp:199-325,
+// without the weights, whose two signs cancel). With g = 0: +-0, the sign of
+// the stored density.
+template <class C>
+inline C gravity_product(C g0, C g1, C g2)
+{
+    return ((g0 * g1 * (g0 - g1)) * ((g0 + g1) * (g0 + g2) * (g0 - g2))) *
+           ((g2 - g1) * (g2 + g1) * g2);
+}
+inline int has_gravity(const double (&g)[3]) { return g[0] != 0 || g[1] != 0 || g[2] != 0; }
 
 }  // namespace lbm
 
@@ -95,6 +108,11 @@ struct lbm_solver {
     const void* xunpack[2];  // fused x-face unpack buffers (LEFT, RIGHT), NULL when off
     void* dd_alt;      // second population buffer of the out-of-place pair pass
     uint32_t* status;  // device word: nonzero after a store out of the storage range
+    // bytes the device had stepped (its counter in lbm_abi.cpp) when this
+    // solver's half-step began, the distances from the half-step before it and
+    // of that one from its own predecessor, and its kernel
+    uint64_t step_mark, step_gap[2];
+    int last_kernel;
 };
 
 namespace lbm {
@@ -103,8 +121,8 @@ void set_error(const std::string& msg);
 int hip_fail(hipError_t e, const char* what);
 
 hipError_t launch_init(const lbm_solver* s, hipStream_t st, int write_flags);
-hipError_t launch_alpha(const lbm_solver* s, const Box& b, hipStream_t st);
-hipError_t launch_beta(const lbm_solver* s, const Box& b, hipStream_t st);
+hipError_t launch_alpha(const lbm_solver* s, const Box& b, int opts, hipStream_t st);
+hipError_t launch_beta(const lbm_solver* s, const Box& b, int opts, hipStream_t st);
 
 // field: 0 populations (the lattice vectors of `mask`; buffers keep all 19
 // planes), 1 velocities (3), 2 densities (1)
@@ -192,9 +210,8 @@ inline bool plane_off32(const lbm_solver* s)
 }
 
 // addr64: the planes need 64-bit element offsets (4 GiB and up); the FP32
-// beta with the fused unpack in 1024-thread workgroups then runs out of its
-// 128 registers per thread and spills (half the step rate at 512^3 forced to
-// 64-bit offsets), so it keeps 512-thread workgroups.
+// beta with the fused unpack keeps 512-thread workgroups there, chosen when
+// the 1024-thread kernel spilled (it needs 85 of its 128 registers now).
 inline int default_launch(int precision, int kernel, bool with_pack, bool wide,
                           bool with_unpack = false, bool addr64 = false)
 {
@@ -223,6 +240,95 @@ inline int default_launch(int precision, int kernel, bool with_pack, bool wide,
         // fused unpack's received loads 256-thread ones are faster
         return kernel == 1 && wide && !with_unpack ? LBM_LAUNCH_BIG : 0;
     }
+}
+
+inline bool is_full(const lbm_solver* s, const Box& b)
+{
+    return b.ox == 0 && b.oy == 0 && b.oz == 0 && b.bx == s->size_h[0] &&
+           b.by == s->size_h[1] && b.bz == s->size_h[2];
+}
+
+// Bytes a half-step of the whole domain reads and writes in place.
+inline uint64_t resident_bytes(const lbm_solver* s)
+{
+    const uint64_t out = (s->p.store_densities ? 1 : 0) + (s->p.store_velocities ? 3 : 0);
+    return (uint64_t)s->n * (19 * s->elem_bytes + 1 + out * s->out_bytes);
+}
+
+// Launch options of a whole-domain step without face work whose kernel the
+// caller has not set. What decides is whether the state still lies in a cache
+// when the step starts: near and far are the lesser and the greater of the
+// bytes the device stepped between this half-step and the solver's last, and
+// between that one and its predecessor. Times are us for an alpha and a beta.
+//  * Own bytes up to about the 8 L2s (4 MiB each): every workgroup is resident
+//    at once, no cap on the waves, no renumbering (62^3 FP32, 22 MB: 13.5
+//    against 15.9 with the streaming options; FP64 25.9 against 30.9).
+//  * All within the 256 MB Infinity Cache (one cavity stepped again and again):
+//    alpha cached and uncapped, beta with one contiguous range of cells per
+//    XCD, whose L2 then serves the lines that neighbouring workgroups share:
+//    104^3 FP32 57.5 against 67-74, 140^3 129 against 147-150, FP64 112^3 134
+//    against 163, F16S 180^3 143 against 149. Level at 267 MB, 11 % slower at
+//    323 MB (three solvers in turn that need 254-258 MB together still gain).
+//  * Only the state itself fits (a few steps, then another solver's turn): the
+//    XCD map loses (130^3 FP32 137-139 against 124-126), cached launches
+//    without it win, FP32 beta at 3 waves per SIMD (124.5 against 126.8 without
+//    a cap), 16-bit beta in 1024-thread workgroups (F16S 150^3 101 against
+//    105-110).
+//  * Otherwise the populations stream from HBM: FP32 / FP64 alpha nontemporal
+//    at 2 waves per SIMD. FP32 beta at 2 waves, in 256-thread workgroups with
+//    other solvers in between (200^3 469, other shapes 473-481); stepped alone
+//    up to 640 MB with the XCD map (160^3 222 against 232-238), then in
+//    1024-thread workgroups (220^3 587 against 600-605), and from 1.6 GB
+//    through LDS (300^3 1502 against 1514-1530, 512^3 7440 against 7585). FP64:
+//    to 400 MB the cached options still win (130^3 257 against 269-286), to
+//    800 MB beta at 2 waves (150^3 409 against 414), then through LDS (256^3
+//    1917 against 1956). F16S / BF16S beta in 1024-thread workgroups, one per
+//    CU (512^3 3970 against 4150 with two, 220^3 327 against 344), F16C, with
+//    more integer work per cell, two (512^3 4055 against 4285 in 256-thread
+//    ones); round robin over solvers that would each fit the cache 16-bit
+//    alpha nontemporal and beta with the XCD map (eight 130^3 F16S 729 against
+//    754-774).
+constexpr int kCapWaves5 = 1 << 16;   // at most 5 waves per SIMD, 256-thread workgroups
+
+inline int step_options(const lbm_solver* s, int kernel, uint64_t near, uint64_t far)
+{
+    constexpr uint64_t MB = 1ull << 20, kL2 = 40 * MB, kCache = 260 * MB;
+    const uint64_t own = resident_bytes(s);
+    if (own <= kL2)
+        return 0;
+    near = near > own ? near : own;
+    far = far > own ? far : own;
+    const int p = s->p.precision;
+    const bool half = p != LBM_F32 && p != LBM_F64;
+    if (near <= kCache) {
+        if (kernel == 0)
+            return 0;
+        if (far > 300 * MB)
+            return half ? LBM_LAUNCH_BIG : p == LBM_F32 ? LBM_LAUNCH_WAVES3 : 0;
+        return LBM_LAUNCH_XCD_REMAP | (p == LBM_F32   ? LBM_LAUNCH_WAVES2
+                                       : p == LBM_F64 ? LBM_LAUNCH_WAVES3
+                                                      : kCapWaves5);
+    }
+    if (half) {
+        if (own <= kCache)
+            return (kernel == 0 ? LBM_LAUNCH_NONTEMPORAL : LBM_LAUNCH_XCD_REMAP) |
+                   LBM_LAUNCH_WAVES4;
+        if (p == LBM_F16C)
+            return kernel == 0 ? 0 : LBM_LAUNCH_BIG;
+        return LBM_LAUNCH_WAVES4 | (kernel == 0 ? 0 : LBM_LAUNCH_BIG);
+    }
+    if (p == LBM_F64 && own > kCache && own <= 400 * MB)
+        return kernel == 0 ? 0 : LBM_LAUNCH_XCD_REMAP | LBM_LAUNCH_WAVES3;
+    if (kernel == 0)
+        return LBM_LAUNCH_NONTEMPORAL | LBM_LAUNCH_WAVES2;
+    if (p == LBM_F64)
+        return LBM_LAUNCH_WAVES2 | (own <= 800 * MB ? 0 : LBM_LAUNCH_LDS);
+    if (own >= 1600 * MB)
+        return LBM_LAUNCH_LDS | LBM_LAUNCH_WAVES4;
+    if (far > own + own / 4)   // other solvers in between
+        return LBM_LAUNCH_WAVES2;
+    return own < 640 * MB ? LBM_LAUNCH_XCD_REMAP | LBM_LAUNCH_WAVES3
+                          : LBM_LAUNCH_BIG | LBM_LAUNCH_WAVES4;
 }
 
 // ||u - u_prev|| / ||u|| from the two FP64 sums; a non-finite state gives NaN

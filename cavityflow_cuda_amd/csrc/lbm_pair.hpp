@@ -53,7 +53,8 @@ struct PairDesc {
     int32_t nx, ny, nz;
     int32_t tiles_x, tiles_y, chunks;
     uint32_t tile_begin;
-    double inv_tau, lid, g0, g1, g2;
+    double inv_tau, lid, g0, g1, g2, rest_rho;
+    int32_t gravity;
     uint32_t* status;
 };
 
@@ -108,6 +109,7 @@ struct PairAlphaAcc {
     const S* in;  // the cell's 19 prefetched slots
     PairLds<S, kWin> lds;
     int p, c;
+    __device__ __forceinline__ PairAlphaAcc for_stores() const { return *this; }
     __device__ __forceinline__ S load(int l, int32_t) const { return in[l]; }
     __device__ __forceinline__ void store(int s, int32_t, S v) const { lds.slot(s, p)[c] = v; }
 };
@@ -121,6 +123,7 @@ struct PairBetaAcc {
     S* dst;
     int64_t stride;
     uint32_t id;
+    __device__ __forceinline__ PairBetaAcc for_stores() const { return *this; }
     __device__ __forceinline__ S load(int l, int32_t) const
     {
         return lds.slot(l, z + cz(l))[c + cy(l) * kWX + cx(l)];
@@ -152,6 +155,8 @@ __device__ __forceinline__ StepArgs<C> pair_args(const PairDesc& d)
     a.g0 = (C)d.g0;
     a.g1 = (C)d.g1;
     a.g2 = (C)d.g2;
+    a.gravity = d.gravity;
+    a.rest_rho = (C)d.rest_rho;
     a.store_rho = 0;
     a.store_u = 0;
     a.xpack_on = 0;

@@ -161,7 +161,10 @@ __global__ __launch_bounds__(Shape<SHAPE>::kThreads) void k_beta(StepArgs<typena
         if (gid >= a.cells)
             return;
         const uint32_t id = FULL ? gid : box_cell(a, gid);
-        if (wrap) {
+        if (wrap && OFF32) {
+            const AccWrap32<S> acc{(const char*)a.dd, a.stride, (int32_t)id, a.n};
+            beta_cell<P, XF>(a, id, a.flags[id], acc);
+        } else if (wrap) {
             const Acc64<S, true> acc{(S*)a.dd, a.stride, (int32_t)id, a.n};
             beta_cell<P, XF>(a, id, a.flags[id], acc);
         } else if (OFF32) {
@@ -188,6 +191,7 @@ template <class S>
 struct AccLds {
     S (*tile)[kBlock];
     uint32_t t;
+    __device__ __forceinline__ AccLds for_stores() const { return *this; }
     __device__ __forceinline__ S load(int l, int32_t) const { return tile[l][t]; }
     __device__ __forceinline__ void store(int l, int32_t, S v) const { tile[l][t] = v; }
 };
@@ -205,7 +209,7 @@ __global__ __launch_bounds__(kBlock) void k_beta_lds(StepArgs<typename P::C> a)
         // uniform per workgroup: no barrier on this path
         const uint32_t id = b + t;
         if (id < a.cells) {
-            const Acc64<S, true> acc{(S*)a.dd, a.stride, (int32_t)id, a.n};
+            const AccWrap32<S> acc{(const char*)a.dd, a.stride, (int32_t)id, a.n};
             beta_cell<P, XF>(a, id, a.flags[id], acc);
         }
         return;
@@ -272,13 +276,17 @@ static StepArgs<typename P::C> make_args(const lbm_solver* s, const Box& b)
     a.oy = b.oy;
     a.oz = b.oz;
     a.cells = b.cells();
-    a.div_bx = FastDiv((uint32_t)b.bx);
-    a.div_by = FastDiv((uint32_t)b.by);
+    if (!is_full(s, b)) {   // whole-domain kernels take the cell index as it is
+        a.div_bx = FastDiv((uint32_t)b.bx);
+        a.div_by = FastDiv((uint32_t)b.by);
+    }
     a.inv_tau = (C)s->p.inv_tau;
     a.lid = (C)s->p.lid_velocity;
     a.g0 = (C)s->p.gravitation[0];
     a.g1 = (C)s->p.gravitation[1];
     a.g2 = (C)s->p.gravitation[2];
+    a.gravity = has_gravity(s->p.gravitation);
+    a.rest_rho = gravity_product(a.g0, a.g1, a.g2);
     a.store_rho = s->p.store_densities;
     a.store_u = s->p.store_velocities;
     a.xcd = 0;
@@ -287,19 +295,14 @@ static StepArgs<typename P::C> make_args(const lbm_solver* s, const Box& b)
     a.xunpack[0] = (const C*)s->xunpack[0];
     a.xunpack[1] = (const C*)s->xunpack[1];
     a.xpack_on = (s->xpack[0] || s->xpack[1] || s->xunpack[0] || s->xunpack[1]) ? 1 : 0;
-    a.div_nx = FastDiv((uint32_t)s->size_h[0]);
+    if (a.xpack_on)
+        a.div_nx = FastDiv((uint32_t)s->size_h[0]);
     a.ny = s->size_h[1];
     a.fcells = s->size_h[1] * s->size_h[2];
     a.status = s->status;
     for (int l = 0; l < kQ; l++)
         a.plane[l] = (const char*)s->dd + (int64_t)l * s->stride * (int64_t)sizeof(typename P::S);
     return a;
-}
-
-static bool is_full(const lbm_solver* s, const Box& b)
-{
-    return b.ox == 0 && b.oy == 0 && b.oz == 0 && b.bx == s->size_h[0] &&
-           b.by == s->size_h[1] && b.bz == s->size_h[2];
 }
 
 template <class P>
@@ -321,6 +324,7 @@ static hipError_t init_t(const lbm_solver* s, hipStream_t st, int write_flags)
 // i.e. 4 (3, 2) waves per SIMD. Fewer resident waves means fewer concurrent
 // 19-plane streams, which the in-place FP32 steps turn into higher DRAM
 // efficiency.
+constexpr size_t kWaves5Lds = 27 * 1024 + 512;   // kCapWaves5
 constexpr size_t kWaves4Lds = 33 * 1024;
 constexpr size_t kWaves3Lds = 41 * 1024;
 constexpr size_t kWaves2Lds = 54 * 1024;
@@ -346,7 +350,8 @@ static void launch_shape(const lbm_solver* s, const StepArgs<typename P::C>& a, 
                                                                              : 0)
                        : (opts & LBM_LAUNCH_WAVES2) ? kWaves2Lds
                        : (opts & LBM_LAUNCH_WAVES3) ? kWaves3Lds
-                       : (opts & LBM_LAUNCH_WAVES4) ? kWaves4Lds : 0;
+                       : (opts & LBM_LAUNCH_WAVES4) ? kWaves4Lds
+                       : (opts & kCapWaves5)        ? kWaves5Lds : 0;
     const dim3 grid(blocks), block(G::kThreads);
     if (!plane_off32(s) || (opts & LBM_LAUNCH_ADDR64))
         hipLaunchKernelGGL((K<P, FULL, false, false, SHAPE, XF>::kernel), grid, block, lds, st, a);
@@ -398,14 +403,14 @@ struct BetaK {
 };
 
 template <class P>
-static hipError_t alpha_t(const lbm_solver* s, const Box& b, hipStream_t st)
+static hipError_t alpha_t(const lbm_solver* s, const Box& b, int opts, hipStream_t st)
 {
     auto a = make_args<P>(s, b);
-    a.xcd = (s->launch[0] & LBM_LAUNCH_XCD_REMAP) ? 1 : 0;
+    a.xcd = (opts & LBM_LAUNCH_XCD_REMAP) ? 1 : 0;
     if (is_full(s, b))
-        launch_variant<P, AlphaK, true>(s, a, s->launch[0], st);
+        launch_variant<P, AlphaK, true>(s, a, opts, st);
     else
-        launch_variant<P, AlphaK, false>(s, a, s->launch[0], st);
+        launch_variant<P, AlphaK, false>(s, a, opts, st);
     return hipGetLastError();
 }
 
@@ -438,23 +443,22 @@ static void launch_beta_lds(const lbm_solver* s, const StepArgs<typename P::C>& 
 }
 
 template <class P>
-static hipError_t beta_t(const lbm_solver* s, const Box& b, hipStream_t st)
+static hipError_t beta_t(const lbm_solver* s, const Box& b, int opts, hipStream_t st)
 {
     auto a = make_args<P>(s, b);
-    a.xcd = (s->launch[1] & LBM_LAUNCH_XCD_REMAP) ? 1 : 0;
+    a.xcd = (opts & LBM_LAUNCH_XCD_REMAP) ? 1 : 0;
     // beta reads and writes plane l at id + c_l: fold the shift into the base
     for (int l = 0; l < kQ; l++)
         a.plane[l] += (int64_t)(cx(l) + cy(l) * a.nx + cz(l) * a.nxy) *
                       (int64_t)sizeof(typename P::S);
-    const int opts = s->launch[1];
     if ((opts & LBM_LAUNCH_LDS) && is_full(s, b) && plane_off32(s) && !(opts & LBM_LAUNCH_ADDR64)) {
         launch_beta_lds<P>(s, a, opts, st);
         return hipGetLastError();
     }
     if (is_full(s, b))
-        launch_variant<P, BetaK, true>(s, a, s->launch[1], st);
+        launch_variant<P, BetaK, true>(s, a, opts, st);
     else
-        launch_variant<P, BetaK, false>(s, a, s->launch[1], st);
+        launch_variant<P, BetaK, false>(s, a, opts, st);
     return hipGetLastError();
 }
 
@@ -472,13 +476,13 @@ hipError_t launch_init(const lbm_solver* s, hipStream_t st, int write_flags)
 {
     LBM_DISPATCH(init_t, s, st, write_flags)
 }
-hipError_t launch_alpha(const lbm_solver* s, const Box& b, hipStream_t st)
+hipError_t launch_alpha(const lbm_solver* s, const Box& b, int opts, hipStream_t st)
 {
-    LBM_DISPATCH(alpha_t, s, b, st)
+    LBM_DISPATCH(alpha_t, s, b, opts, st)
 }
-hipError_t launch_beta(const lbm_solver* s, const Box& b, hipStream_t st)
+hipError_t launch_beta(const lbm_solver* s, const Box& b, int opts, hipStream_t st)
 {
-    LBM_DISPATCH(beta_t, s, b, st)
+    LBM_DISPATCH(beta_t, s, b, opts, st)
 }
 
 }  // namespace lbm

@@ -66,9 +66,12 @@ struct StoreF16S : Unchecked<StoreF16S> {
     {
         return __builtin_fmaf((float)v, 1.0f / kScale, weight<float>(l));
     }
+    // v - w rounds once and scales by a power of two, as the fused form does
+    // (v * 2^12 - w * 2^12 rounded once to FP32, then to FP16): one
+    // mixed-precision FMA instead of a subtraction and the FMA
     __device__ static __forceinline__ S store(C v, int l)
     {
-        return (_Float16)((v - weight<float>(l)) * kScale);
+        return (_Float16)__builtin_fmaf(v, kScale, -(weight<float>(l) * kScale));
     }
     __device__ static __forceinline__ S store_checked(C v, int l, uint32_t&) { return store(v, l); }
 };

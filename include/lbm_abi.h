@@ -173,7 +173,13 @@ int lbm_simulation_step_beta(lbm_solver* solver, const int origin[3], const int 
                              hipStream_t stream);
 
 /* Launch variants of the step kernels; they change speed, never results.
- * kernel: 0 = alpha, 1 = beta. Defaults (measured on MI355X): F32 beta
+ * kernel: 0 = alpha, 1 = beta. Options set here are the ones every launch of
+ * that kernel takes. Whole-domain steps of a kernel that was not set, without
+ * a step pack or unpack, choose theirs at each launch by the bytes the device
+ * has stepped since this solver's previous half-step (whether its state can
+ * still lie in the L2s or the Infinity Cache) and by the domain's own bytes.
+ * Box steps and steps with face work of a kernel that was not set take the
+ * defaults that lbm_get_launch_options reports (measured on MI355X): F32 beta
  * WIDE | WAVES2 on domains of 6 Mi cells or more (halo included: from 183^3
  * interior cells), BIG | WAVES4 there with a step pack or unpack
  * (lbm_set_step_pack / lbm_set_step_unpack) except WIDE | WAVES3 with an
@@ -207,10 +213,7 @@ enum lbm_launch_option {
     LBM_LAUNCH_BIG = 256         /* 1024-thread workgroups, one cell per thread
                                     (wins over WIDE; a workgroup alone fills 4
                                     waves per SIMD, so any WAVES cap holds one per
-                                    CU; single-domain kernels only; beta spills
-                                    registers in this shape for F64, and with a
-                                    step unpack and 64-bit indexing for the
-                                    other formats) */
+                                    CU; single-domain kernels only) */
 };
 int lbm_set_launch_options(lbm_solver* solver, int kernel, int options);
 int lbm_get_launch_options(const lbm_solver* solver, int kernel, int* options);
