@@ -468,6 +468,11 @@ typedef struct lbm_batch_tuning {
                               Not with pairs. */
 } lbm_batch_tuning;
 
+/* A batch whose tuning was neither set nor autotuned runs 256-thread tiles as
+ * lbm_batch_get_tuning reports them, but in groups of at most 224 MiB, with
+ * launch options chosen by whether a group's state stays in the last-level
+ * cache between its half-steps. */
+
 int lbm_batch_create(lbm_solver* const* members, int count, lbm_batch** out);
 int lbm_batch_destroy(lbm_batch* batch);
 int lbm_batch_size(const lbm_batch* batch);
