@@ -10,6 +10,7 @@
 #include <cstdio>
 #include <cstring>
 #include <limits>
+#include <mutex>
 #include <string>
 #include <utility>
 #include <vector>
@@ -114,6 +115,66 @@ int ensure_staging(lbm_solver* s, size_t bytes)
         return LBM_ERR_NOMEM;
     }
     s->staging_bytes = bytes;
+    return LBM_OK;
+}
+
+// Pinned host memory that the reductions' last kernel writes its 5 values to,
+// one slot per solver: a copy from the device into pageable memory behind every
+// reduction took 10-20 us more. One block per process, allocated with the first
+// solver; a slot goes back when its solver is destroyed, and solvers beyond
+// the last slot copy from the device.
+constexpr int kResultSlots = 1024;
+constexpr int kResultDoubles = 8;   // a cache line each
+std::mutex g_results_mutex;
+double* g_results = nullptr;
+std::vector<int> g_free_results;
+
+double* take_result_slot()
+{
+    std::lock_guard<std::mutex> lock(g_results_mutex);
+    if (!g_results) {
+        void* p = nullptr;
+        if (hipHostMalloc(&p, kResultSlots * kResultDoubles * sizeof(double),
+                          hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent) !=
+            hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        g_results = (double*)p;
+        for (int i = kResultSlots; i-- > 0;)
+            g_free_results.push_back(i);
+    }
+    if (g_free_results.empty())
+        return nullptr;
+    const int i = g_free_results.back();
+    g_free_results.pop_back();
+    return g_results + (size_t)i * kResultDoubles;
+}
+
+void give_result_slot(double* slot)
+{
+    if (!slot)
+        return;
+    std::lock_guard<std::mutex> lock(g_results_mutex);
+    g_free_results.push_back((int)((slot - g_results) / kResultDoubles));
+}
+
+// Where a reduction's last kernel writes its values, and the wait for them.
+double* result_target(lbm_solver* s)
+{
+    return s->result ? s->result : s->partials + kReduceBlocks * 5;
+}
+
+int read_result(lbm_solver* s, double* out, hipStream_t stream)
+{
+    if (!s->result)
+        LBM_HIP(hipMemcpyAsync(out, s->partials + kReduceBlocks * 5, 5 * sizeof(double),
+                               hipMemcpyDeviceToHost, stream),
+                "D2H copy");
+    LBM_HIP(hipStreamSynchronize(stream), "hipStreamSynchronize");
+    if (s->result)
+        for (int k = 0; k < 5; k++)
+            out[k] = ((volatile double*)s->result)[k];
     return LBM_OK;
 }
 
@@ -439,6 +500,7 @@ int lbm_create(const lbm_params* params, lbm_solver** out)
         return fail(LBM_ERR_NOMEM, "cannot allocate velocities");
     if (hipMalloc((void**)&s->partials, kPartialsBytes) != hipSuccess)
         return fail(LBM_ERR_NOMEM, "cannot allocate reduction buffer");
+    s->result = take_result_slot();
     // the overflow word after the partials; the init kernel clears it
     s->status = (uint32_t*)(s->partials + (kReduceBlocks + 1) * 5);
     hipError_t e = launch_init(s, nullptr, 1);
@@ -467,6 +529,7 @@ int lbm_destroy(lbm_solver* s)
     for (void* b : bufs)
         if (b)
             (void)hipFree(b);
+    give_result_slot(s->result);
     delete s;
     return LBM_OK;
 }
@@ -1026,12 +1089,8 @@ int lbm_reduce_box(lbm_solver* s, const int origin[3], const int size[3], double
     }
     if ((rc = set_device(s)))
         return rc;
-    double* res = s->partials + kReduceBlocks * 5;
-    LBM_HIP(launch_reduce_box(s, b, s->partials, res, stream), "reduce kernel");
-    LBM_HIP(hipMemcpyAsync(out, res, 5 * sizeof(double), hipMemcpyDeviceToHost, stream),
-            "D2H copy");
-    LBM_HIP(hipStreamSynchronize(stream), "hipStreamSynchronize");
-    return LBM_OK;
+    LBM_HIP(launch_reduce_box(s, b, s->partials, result_target(s), stream), "reduce kernel");
+    return read_result(s, out, stream);
 }
 
 int lbm_reduce_boxes_noalloc(lbm_solver* const* solvers, const int* origins, const int* sizes,
@@ -1095,12 +1154,10 @@ int lbm_residual(lbm_solver* s, int layout, double* residual, hipStream_t stream
         LBM_HIP(hipMemset(s->residual_prev, 0, bytes), "hipMemset");
         s->residual_valid = 0;
     }
-    double* res = s->partials + kReduceBlocks * 5;
     double host[5];
-    LBM_HIP(launch_residual(s, layout, s->partials, res, stream), "residual kernel");
-    LBM_HIP(hipMemcpyAsync(host, res, 5 * sizeof(double), hipMemcpyDeviceToHost, stream),
-            "D2H copy");
-    LBM_HIP(hipStreamSynchronize(stream), "hipStreamSynchronize");
+    LBM_HIP(launch_residual(s, layout, s->partials, result_target(s), stream), "residual kernel");
+    if ((rc = read_result(s, host, stream)))
+        return rc;
     *residual = first_residual(s->residual_valid, host[0], host[1]);
     s->residual_valid = 1;
     return LBM_OK;

@@ -100,6 +100,7 @@ struct lbm_solver {
     void* staging;     // device staging for host copies
     size_t staging_bytes;
     double* partials;  // reduction partials (kReduceBlocks * 5) followed by 5 results
+    double* result;    // pinned host memory for 5 results, NULL when none was free
     void* residual_prev;  // momentum saved by lbm_residual, 3 planes of the compute type
     int residual_valid;
     int launch[2];     // LBM_LAUNCH_* options of the alpha and beta kernels
@@ -177,7 +178,7 @@ hipError_t launch_residual_members(int precision, const ResidualMember* mem, int
                                    int layout, double* partials, double* out_dev,
                                    hipStream_t st);
 
-constexpr int kReduceBlocks = 1024;
+constexpr int kReduceBlocks = 2048;   // at most: 8 workgroups on each of 256 CUs
 // Per-solver reduction buffer: kReduceBlocks * 5 partial sums, 5 results,
 // then the solver's overflow word (lbm_solver::status).
 constexpr size_t kPartialsBytes = (size_t)(kReduceBlocks + 1) * 5 * sizeof(double) + 64;

@@ -1,6 +1,16 @@
 // FP64 reductions over the population field: total mass / momentum of a box
 // and the steady-state residual ||u - u_prev||_2 / ||u||_2. Two passes with a
-// fixed block count and a fixed final order, so results are deterministic.
+// block count fixed by the cells and a fixed final order, so results are
+// deterministic.
+//
+// Both are bound by the 19-plane read. One cell per thread and iteration in 47
+// to 64 VGPRs leaves room for 8 waves per SIMD, which kReduceBlocks fills;
+// states larger than the Infinity Cache are read with nontemporal loads (NT; a
+// bare 19-plane read runs 7.18 TB/s with them, 6.44 without), smaller ones
+// with cached loads, so that they stay for the steps around the reduction.
+// 384^3 FP32: box sums 757 us with 4 waves and cached loads, 674 (6.5 TB/s)
+// now; residual, which also rewrites the last momentum, 1194 and 1102.
+// k_moments gains nothing from nontemporal accesses (977 us, 988 with them).
 #include "lbm_d3q19.hpp"
 #include "lbm_internal.hpp"
 #include "lbm_storage.hpp"
@@ -51,6 +61,27 @@ struct RedArgs {
     const uint32_t* status;   // the solver's overflow word
 };
 
+template <bool NT, class T>
+__device__ __forceinline__ T read_stream(const T* p)
+{
+    return NT ? __builtin_nontemporal_load(p) : *p;
+}
+template <bool NT, class T>
+__device__ __forceinline__ void write_stream(T* p, T v)
+{
+    if (NT)
+        __builtin_nontemporal_store(v, p);
+    else
+        *p = v;
+}
+
+// Blocks that share the cells: small domains leave no block without one.
+__host__ __device__ __forceinline__ uint32_t reduce_blocks(uint32_t cells)
+{
+    const uint32_t b = (cells + kRedBlock - 1) / kRedBlock;
+    return b < (uint32_t)kReduceBlocks ? b : (uint32_t)kReduceBlocks;
+}
+
 // A state with a population store out of its storage range (F16C) has no
 // meaningful sums: they become NaN, as a non-finite state's are.
 __device__ __forceinline__ bool poisoned(const uint32_t* status)
@@ -60,7 +91,7 @@ __device__ __forceinline__ bool poisoned(const uint32_t* status)
 
 // Block `block` of `nblocks` strides over the cells of the box; its sums go to
 // partials[block].
-template <class P>
+template <class P, bool NT>
 __device__ __forceinline__ void reduce_box_block(const typename P::S* __restrict__ dd,
                                                  const RedArgs& a, uint32_t block,
                                                  uint32_t nblocks, double* partials)
@@ -76,7 +107,7 @@ __device__ __forceinline__ void reduce_box_block(const typename P::S* __restrict
                                        a.ox + (int32_t)x);
 #pragma unroll
         for (int l = 0; l < kQ; l++) {
-            const double f = (double)P::load(dd[(int64_t)l * a.stride + id], l);
+            const double f = (double)P::load(read_stream<NT>(dd + (int64_t)l * a.stride + id), l);
             acc[0] += f;
             acc[1] += cx(l) * f;
             acc[2] += cy(l) * f;
@@ -90,11 +121,11 @@ __device__ __forceinline__ void reduce_box_block(const typename P::S* __restrict
     block_store(acc, partials, block);
 }
 
-template <class P>
+template <class P, bool NT>
 __global__ __launch_bounds__(kRedBlock) void k_reduce_box(const typename P::S* __restrict__ dd,
                                                           RedArgs a, double* partials)
 {
-    reduce_box_block<P>(dd, a, blockIdx.x, gridDim.x, partials);
+    reduce_box_block<P, NT>(dd, a, blockIdx.x, gridDim.x, partials);
 }
 
 // The box sums of several solvers in one launch: grid.y = member, and member
@@ -113,8 +144,10 @@ __global__ __launch_bounds__(kRedBlock) void k_reduce_boxes(ReduceBoxMembers mem
                                                             double* partials)
 {
     const ReduceBoxMember& m = mem.m[blockIdx.y];
-    reduce_box_block<P>((const typename P::S*)m.dd, m.a, blockIdx.x, gridDim.x,
-                        partials + (size_t)blockIdx.y * gridDim.x * kRedVals);
+    const uint32_t nblocks = reduce_blocks(m.a.cells);
+    if (blockIdx.x < nblocks)
+        reduce_box_block<P, false>((const typename P::S*)m.dd, m.a, blockIdx.x, nblocks,
+                                   partials + (size_t)blockIdx.y * kReduceBlocks * kRedVals);
 }
 
 // Residual over FLUID cells. LAYOUT 0: slot l holds direction l (after beta);
@@ -122,7 +155,7 @@ __global__ __launch_bounds__(kRedBlock) void k_reduce_boxes(ReduceBoxMembers mem
 // with a run-time layout the slot permutation became register-indexed moves
 // that serialise the 19 loads. Block `block` of `nblocks` strides over the
 // cells; its sums go to partials[block].
-template <class P, int LAYOUT>
+template <class P, int LAYOUT, bool NT>
 __device__ __forceinline__ void residual_block(const typename P::S* __restrict__ dd,
                                                const uint8_t* __restrict__ flags,
                                                typename P::C* __restrict__ prev,
@@ -142,9 +175,10 @@ __device__ __forceinline__ void residual_block(const typename P::S* __restrict__
         C d[kQ];
 #pragma unroll
         for (int l = 0; l < kQ; l++) {
-            d[LAYOUT ? opp(l) : l] = P::load(dd[(int64_t)l * stride + id], l);
+            d[LAYOUT ? opp(l) : l] = P::load(read_stream<NT>(dd + (int64_t)l * stride + id), l);
         }
-        const C p0 = prev[id], p1 = prev[stride + id], p2 = prev[2 * stride + id];
+        const C p0 = read_stream<NT>(prev + id), p1 = read_stream<NT>(prev + stride + id),
+                p2 = read_stream<NT>(prev + 2 * stride + id);
         // empty statements that read every loaded value: the compiler cannot
         // sink the loads below the flag test into the FLUID path
 #pragma unroll
@@ -159,16 +193,16 @@ __device__ __forceinline__ void residual_block(const typename P::S* __restrict__
         acc[0] += fluid ? dx * dx + dy * dy + dz * dz : 0.0;
         acc[1] += fluid ? (double)ux * ux + (double)uy * uy + (double)uz * uz : 0.0;
         acc[2] += fluid ? 1.0 : 0.0;
-        prev[id] = fluid ? ux : p0;
-        prev[stride + id] = fluid ? uy : p1;
-        prev[2 * stride + id] = fluid ? uz : p2;
+        write_stream<NT>(prev + id, fluid ? ux : p0);
+        write_stream<NT>(prev + stride + id, fluid ? uy : p1);
+        write_stream<NT>(prev + 2 * stride + id, fluid ? uz : p2);
     }
     if (poisoned(status))
         acc[0] = acc[1] = __builtin_nan("");
     block_store(acc, partials, block);
 }
 
-template <class P, int LAYOUT>
+template <class P, int LAYOUT, bool NT>
 __global__ __launch_bounds__(kRedBlock) void k_residual(const typename P::S* __restrict__ dd,
                                                         const uint8_t* __restrict__ flags,
                                                         typename P::C* __restrict__ prev,
@@ -176,8 +210,8 @@ __global__ __launch_bounds__(kRedBlock) void k_residual(const typename P::S* __r
                                                         double* partials,
                                                         const uint32_t* status)
 {
-    residual_block<P, LAYOUT>(dd, flags, prev, stride, n, blockIdx.x, gridDim.x, partials,
-                              status);
+    residual_block<P, LAYOUT, NT>(dd, flags, prev, stride, n, blockIdx.x, gridDim.x, partials,
+                                  status);
 }
 
 // The residual of many solvers in one launch: grid.y = member, and member m's
@@ -189,9 +223,13 @@ __global__ __launch_bounds__(kRedBlock) void k_residual_members(const ResidualMe
                                                                 double* partials)
 {
     const ResidualMember& m = mem[blockIdx.y];
-    residual_block<P, LAYOUT>((const typename P::S*)m.dd, m.flags, (typename P::C*)m.prev,
-                              m.stride, m.n, blockIdx.x, gridDim.x,
-                              partials + (size_t)blockIdx.y * gridDim.x * kRedVals, m.status);
+    const uint32_t nblocks = reduce_blocks(m.n);
+    if (blockIdx.x < nblocks)
+        residual_block<P, LAYOUT, false>((const typename P::S*)m.dd, m.flags,
+                                         (typename P::C*)m.prev, m.stride, m.n, blockIdx.x,
+                                         nblocks,
+                                         partials + (size_t)blockIdx.y * kReduceBlocks * kRedVals,
+                                         m.status);
 }
 
 // Density and momentum of every cell of a box, computed from the populations
@@ -225,24 +263,57 @@ __global__ __launch_bounds__(kRedBlock) void k_moments(const typename P::S* __re
     dst[3 * (int64_t)a.cells + gid] = uz;
 }
 
-// Sum of the per-block partials in a fixed order (lane i adds blocks i, i + 64,
-// ... in turn, then the butterfly over the wave): the same bits on every call,
-// in a few microseconds instead of one lane walking all blocks.
-// grid.x > 1: one slice of nblocks partials and one output per workgroup.
-__global__ __launch_bounds__(64) void k_finalize(const double* partials, int nblocks,
-                                                 double* out)
+// Sums of the per-block partials in a fixed order: wave k of the workgroup sums
+// value k, lane i adding blocks i, i + 64, ... in turn, then the butterfly over
+// the wave. All of a lane's loads are issued before the first addition: 4.2 us
+// where a single wave that walked the five values in a loop took 16.
+constexpr int kFinalThreads = 64 * kRedVals;
+__device__ __forceinline__ void finalize(const double* partials, uint32_t nblocks, double* out)
 {
-    partials += (size_t)blockIdx.x * nblocks * kRedVals;
-    out += (size_t)blockIdx.x * kRedVals;
+    constexpr int kPerLane = kReduceBlocks / 64;
+    const uint32_t lane = threadIdx.x & 63, k = threadIdx.x >> 6;
+    double v[kPerLane];
 #pragma unroll
-    for (int k = 0; k < kRedVals; k++) {
-        double t = 0.0;
-        for (int b = threadIdx.x; b < nblocks; b += 64)
-            t += partials[b * kRedVals + k];
-        t = wave_sum(t);
-        if (threadIdx.x == 0)
-            out[k] = t;
+    for (int i = 0; i < kPerLane; i++) {
+        const uint32_t b = lane + 64 * i;
+        v[i] = b < nblocks ? partials[b * kRedVals + k] : 0.0;
     }
+    double t = 0.0;
+#pragma unroll
+    for (int i = 0; i < kPerLane; i++)
+        t += v[i];
+    t = wave_sum(t);
+    if (lane == 0)
+        out[k] = t;
+}
+
+__global__ __launch_bounds__(kFinalThreads) void k_finalize(const double* partials,
+                                                            uint32_t cells, double* out)
+{
+    finalize(partials, reduce_blocks(cells), out);
+}
+
+// One slice of kReduceBlocks partials and one output per workgroup.
+__global__ __launch_bounds__(kFinalThreads) void k_finalize_members(const ResidualMember* mem,
+                                                                    const double* partials,
+                                                                    double* out)
+{
+    finalize(partials + (size_t)blockIdx.x * kReduceBlocks * kRedVals,
+             reduce_blocks(mem[blockIdx.x].n), out + (size_t)blockIdx.x * kRedVals);
+}
+
+__global__ __launch_bounds__(kFinalThreads) void k_finalize_boxes(ReduceBoxMembers mem,
+                                                                  const double* partials,
+                                                                  double* out)
+{
+    finalize(partials + (size_t)blockIdx.x * kReduceBlocks * kRedVals,
+             reduce_blocks(mem.m[blockIdx.x].a.cells), out + (size_t)blockIdx.x * kRedVals);
+}
+
+// Whether the box's populations exceed what the Infinity Cache keeps.
+static bool streams(const lbm_solver* s, uint32_t cells)
+{
+    return (uint64_t)cells * kQ * (uint64_t)s->elem_bytes > (260ull << 20);
 }
 
 static RedArgs red_args(const lbm_solver* s, const Box& b)
@@ -266,27 +337,39 @@ static hipError_t reduce_box_t(const lbm_solver* s, const Box& b, double* partia
                                double* out, hipStream_t st)
 {
     const RedArgs a = red_args(s, b);
-    hipLaunchKernelGGL(k_reduce_box<P>, dim3(kReduceBlocks), dim3(kRedBlock), 0, st,
-                       (const typename P::S*)s->dd, a, partials);
-    hipLaunchKernelGGL(k_finalize, dim3(1), dim3(64), 0, st, partials, kReduceBlocks, out);
+    const dim3 grid(reduce_blocks(a.cells));
+    if (streams(s, a.cells))
+        hipLaunchKernelGGL((k_reduce_box<P, true>), grid, dim3(kRedBlock), 0, st,
+                           (const typename P::S*)s->dd, a, partials);
+    else
+        hipLaunchKernelGGL((k_reduce_box<P, false>), grid, dim3(kRedBlock), 0, st,
+                           (const typename P::S*)s->dd, a, partials);
+    hipLaunchKernelGGL(k_finalize, dim3(1), dim3(kFinalThreads), 0, st, partials, a.cells, out);
     return hipGetLastError();
+}
+
+template <class P, int LAYOUT, bool NT>
+static void residual_launch(const lbm_solver* s, double* partials, hipStream_t st)
+{
+    hipLaunchKernelGGL((k_residual<P, LAYOUT, NT>), dim3(reduce_blocks((uint32_t)s->n)),
+                       dim3(kRedBlock), 0, st, (const typename P::S*)s->dd, s->flags,
+                       (typename P::C*)s->residual_prev, s->stride, (uint32_t)s->n, partials,
+                       s->status);
 }
 
 template <class P>
 static hipError_t residual_t(const lbm_solver* s, int layout, double* partials, double* out,
                              hipStream_t st)
 {
+    const bool nt = streams(s, (uint32_t)s->n);
     if (layout)
-        hipLaunchKernelGGL((k_residual<P, 1>), dim3(kReduceBlocks), dim3(kRedBlock), 0, st,
-                           (const typename P::S*)s->dd, s->flags,
-                           (typename P::C*)s->residual_prev, s->stride, (uint32_t)s->n,
-                           partials, s->status);
+        nt ? residual_launch<P, 1, true>(s, partials, st)
+           : residual_launch<P, 1, false>(s, partials, st);
     else
-        hipLaunchKernelGGL((k_residual<P, 0>), dim3(kReduceBlocks), dim3(kRedBlock), 0, st,
-                           (const typename P::S*)s->dd, s->flags,
-                           (typename P::C*)s->residual_prev, s->stride, (uint32_t)s->n,
-                           partials, s->status);
-    hipLaunchKernelGGL(k_finalize, dim3(1), dim3(64), 0, st, partials, kReduceBlocks, out);
+        nt ? residual_launch<P, 0, true>(s, partials, st)
+           : residual_launch<P, 0, false>(s, partials, st);
+    hipLaunchKernelGGL(k_finalize, dim3(1), dim3(kFinalThreads), 0, st, partials, (uint32_t)s->n,
+                       out);
     return hipGetLastError();
 }
 
@@ -341,7 +424,8 @@ static hipError_t residual_members_t(const ResidualMember* mem, int count, int l
     else
         hipLaunchKernelGGL((k_residual_members<P, 0>), dim3(kReduceBlocks, count),
                            dim3(kRedBlock), 0, st, mem, partials);
-    hipLaunchKernelGGL(k_finalize, dim3(count), dim3(64), 0, st, partials, kReduceBlocks, out);
+    hipLaunchKernelGGL(k_finalize_members, dim3(count), dim3(kFinalThreads), 0, st, mem, partials,
+                       out);
     return hipGetLastError();
 }
 
@@ -365,7 +449,7 @@ hipError_t launch_residual_members(int precision, const ResidualMember* mem, int
 // ------------------------------------------------ allocation-free sums ---
 
 // Block partials of lbm_reduce_boxes_noalloc: LBM_NOALLOC_MAX_BOXES slices of
-// kReduceBlocks * kRedVals doubles (640 KiB). Every GPU the library runs on
+// kReduceBlocks * kRedVals doubles (1.25 MiB). Every GPU the library runs on
 // holds its own copy until the process ends. In host code `scratch` names a
 // host-side stand-in, not a device address, so it is never passed to a kernel
 // or a copy: each device's address comes from hipGetSymbolAddress, looked up
@@ -406,7 +490,8 @@ static hipError_t reduce_boxes_t(const lbm_solver* const* s, const Box* b, int c
     }
     hipLaunchKernelGGL(k_reduce_boxes<P>, dim3(kReduceBlocks, count), dim3(kRedBlock), 0, st,
                        mem, partials);
-    hipLaunchKernelGGL(k_finalize, dim3(count), dim3(64), 0, st, partials, kReduceBlocks, out);
+    hipLaunchKernelGGL(k_finalize_boxes, dim3(count), dim3(kFinalThreads), 0, st, mem, partials,
+                       out);
     return hipGetLastError();
 }
 
