@@ -213,35 +213,39 @@ int copy_set(lbm_solver* s, int field, const Box& b, int ncomp, const void* src,
     return LBM_OK;
 }
 
-// Bytes of domains stepped so far on each device (modulo the array): how much
-// passed between two half-steps of one solver says whether its state can still
-// be in the caches. Only launch shapes depend on it, never results.
+// Bytes of domains stepped so far on each device (modulo the arrays), several
+// half-steps of one solver in a row counted once: what passed between two
+// half-steps of a solver says whether its state can still be in the caches.
+// Only launch shapes depend on it, never results.
 std::atomic<uint64_t> g_stepped[64];
+std::atomic<const lbm_solver*> g_last_stepped[64];
 
 // The launch options of a step: the ones set (or the defaults by face work and
 // size), and for whole-domain steps without face work of a kernel the caller
-// has not set, step_options for the bytes stepped between this solver's
-// half-steps.
+// has not set, step_options for the bytes of other solvers stepped since this
+// solver's last half-step.
 int options_of_step(lbm_solver* s, int kernel, const Box& b)
 {
     const bool full = is_full(s, b);
-    const uint64_t bytes = resident_bytes(s) / (uint64_t)s->n * b.cells();
-    const uint64_t now = g_stepped[s->p.device & 63].fetch_add(bytes, std::memory_order_relaxed);
+    const int dev = s->p.device & 63;
+    uint64_t now = g_stepped[dev].load(std::memory_order_relaxed);
     // relaxed atomics: threads that step boxes of one solver side by side may
     // both write the marks
+    const uint64_t gap = now - __atomic_load_n(&s->step_mark, __ATOMIC_RELAXED);
+    const uint64_t gap_before = __atomic_load_n(&s->step_gap, __ATOMIC_RELAXED);
     const int last = __atomic_exchange_n(&s->last_kernel, kernel, __ATOMIC_RELAXED);
-    uint64_t gap = __atomic_load_n(&s->step_gap[0], __ATOMIC_RELAXED);
-    uint64_t gap_before = __atomic_load_n(&s->step_gap[1], __ATOMIC_RELAXED);
-    if (full || kernel != last) {   // box steps of one half-step share its mark
-        gap_before = gap;
-        gap = last < 0 ? 0 : now - __atomic_load_n(&s->step_mark, __ATOMIC_RELAXED);
-        __atomic_store_n(&s->step_gap[1], gap_before, __ATOMIC_RELAXED);
-        __atomic_store_n(&s->step_gap[0], gap, __ATOMIC_RELAXED);
-        __atomic_store_n(&s->step_mark, now, __ATOMIC_RELAXED);
+    if (g_last_stepped[dev].exchange(s, std::memory_order_relaxed) != s) {
+        const uint64_t bytes = resident_bytes(s);
+        now = g_stepped[dev].fetch_add(bytes, std::memory_order_relaxed) + bytes;
     }
+    __atomic_store_n(&s->step_mark, now, __ATOMIC_RELAXED);
+    if (full || kernel != last)   // box steps of one half-step share its gap
+        __atomic_store_n(&s->step_gap, last < 0 ? 0 : gap, __ATOMIC_RELAXED);
     if (!full || s->launch_set[kernel] || s->xpack[0] || s->xpack[1] || s->xunpack[0] ||
         s->xunpack[1] || !plane_off32(s))
         return s->launch[kernel];
+    if (last < 0)
+        return step_options(s, kernel, 0, 0);
     return step_options(s, kernel, std::min(gap, gap_before), std::max(gap, gap_before));
 }
 

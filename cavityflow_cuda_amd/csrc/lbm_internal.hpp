@@ -109,10 +109,9 @@ struct lbm_solver {
     const void* xunpack[2];  // fused x-face unpack buffers (LEFT, RIGHT), NULL when off
     void* dd_alt;      // second population buffer of the out-of-place pair pass
     uint32_t* status;  // device word: nonzero after a store out of the storage range
-    // bytes the device had stepped (its counter in lbm_abi.cpp) when this
-    // solver's half-step began, the distances from the half-step before it and
-    // of that one from its own predecessor, and its kernel
-    uint64_t step_mark, step_gap[2];
+    // the device's counter of stepped bytes (lbm_abi.cpp) at this solver's last
+    // half-step, the bytes of other solvers before that one, and its kernel
+    uint64_t step_mark, step_gap;
     int last_kernel;
 };
 
@@ -259,8 +258,8 @@ inline uint64_t resident_bytes(const lbm_solver* s)
 // Launch options of a whole-domain step without face work whose kernel the
 // caller has not set. What decides is whether the state still lies in a cache
 // when the step starts: near and far are the lesser and the greater of the
-// bytes the device stepped between this half-step and the solver's last, and
-// between that one and its predecessor. Times are us for an alpha and a beta.
+// bytes of other solvers stepped between this half-step and the solver's last,
+// and between that one and its predecessor. Times are us for an alpha and a beta.
 //  * Own bytes up to about the 8 L2s (4 MiB each): every workgroup is resident
 //    at once, no cap on the waves, no renumbering (62^3 FP32, 22 MB: 13.5
 //    against 15.9 with the streaming options; FP64 25.9 against 30.9).
@@ -297,8 +296,8 @@ inline int step_options(const lbm_solver* s, int kernel, uint64_t near, uint64_t
     const uint64_t own = resident_bytes(s);
     if (own <= kL2)
         return 0;
-    near = near > own ? near : own;
-    far = far > own ? far : own;
+    near += own;
+    far += own;
     const int p = s->p.precision;
     const bool half = p != LBM_F32 && p != LBM_F64;
     if (near <= kCache) {
