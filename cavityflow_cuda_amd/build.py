@@ -19,7 +19,7 @@ LIB_NAME = "libcavityflow_hip.so"
 LIB_PATH = os.path.join(HERE, LIB_NAME)
 
 SOURCES = ["lbm_step.hip", "lbm_box.hip", "lbm_reduce.hip", "lbm_batch.hip", "lbm_probe.hip",
-           "lbm_abi.cpp"]
+           "lbm_transfer.cpp", "lbm_abi.cpp"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off",

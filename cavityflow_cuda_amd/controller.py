@@ -357,6 +357,9 @@ class CavityController:
     # -- extraction -----------------------------------------------------------
     def _gather(self, getter, ncomp, dtype=None):
         self.sync()   # the getters copy on the default stream
+        if len(self.solvers) == 1:   # the subdomain's array is the cavity's
+            part = getattr(next(iter(self.solvers.values())), getter)()
+            return part.reshape((ncomp,) + self.size[::-1])
         out = np.empty((ncomp,) + self.size[::-1], dtype=dtype or self.dtype)
         sx, sy, sz = self.sub
         for (i, j, k), s in self.solvers.items():

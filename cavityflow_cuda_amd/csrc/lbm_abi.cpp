@@ -18,6 +18,7 @@
 #include "lbm_abi.h"
 #include "lbm_d3q19.hpp"
 #include "lbm_internal.hpp"
+#include "lbm_transfer.hpp"
 
 namespace lbm {
 
@@ -191,8 +192,7 @@ int copy_get(lbm_solver* s, int field, const Box& b, int ncomp, void* dst, int d
     if (rc)
         return rc;
     LBM_HIP(launch_box_get(s, field, b, s->staging, 0x7FFFFu, st), "box get kernel");
-    LBM_HIP(hipMemcpyAsync(dst, s->staging, bytes, hipMemcpyDeviceToHost, st), "D2H copy");
-    LBM_HIP(hipStreamSynchronize(st), "hipStreamSynchronize");
+    LBM_HIP(transfer(dst, s->staging, bytes, true, st), "D2H copy");
     return LBM_OK;
 }
 
@@ -207,7 +207,7 @@ int copy_set(lbm_solver* s, int field, const Box& b, int ncomp, const void* src,
     int rc = ensure_staging(s, bytes);
     if (rc)
         return rc;
-    LBM_HIP(hipMemcpyAsync(s->staging, src, bytes, hipMemcpyHostToDevice, st), "H2D copy");
+    LBM_HIP(transfer(const_cast<void*>(src), s->staging, bytes, false, st), "H2D copy");
     LBM_HIP(launch_box_set(s, field, b, s->staging, mask, st), "box set kernel");
     LBM_HIP(hipStreamSynchronize(st), "hipStreamSynchronize");
     return LBM_OK;
@@ -678,8 +678,7 @@ int lbm_get_moments(lbm_solver* s, int layout, const int origin[3], const int si
     if ((rc = ensure_staging(s, bytes)))
         return rc;
     LBM_HIP(launch_moments(s, b, layout, s->staging, stream), "moments kernel");
-    LBM_HIP(hipMemcpyAsync(dst, s->staging, bytes, hipMemcpyDeviceToHost, stream), "D2H copy");
-    LBM_HIP(hipStreamSynchronize(stream), "hipStreamSynchronize");
+    LBM_HIP(transfer(dst, s->staging, bytes, true, stream), "D2H copy");
     return LBM_OK;
 }
 
@@ -699,7 +698,7 @@ int lbm_get_flags(lbm_solver* s, const int origin[3], const int size[3], int32_t
     if ((rc = ensure_staging(s, bytes)))
         return rc;
     LBM_HIP(launch_flags_get(s, b, (int32_t*)s->staging, nullptr), "flags get kernel");
-    LBM_HIP(hipMemcpy(dst, s->staging, bytes, hipMemcpyDeviceToHost), "D2H copy");
+    LBM_HIP(transfer(dst, s->staging, bytes, true, nullptr), "D2H copy");
     return LBM_OK;
 }
 
@@ -725,7 +724,8 @@ int lbm_set_flags(lbm_solver* s, const int origin[3], const int size[3], const i
     const size_t bytes = (size_t)cells * sizeof(int32_t);
     if ((rc = ensure_staging(s, bytes)))
         return rc;
-    LBM_HIP(hipMemcpy(s->staging, src, bytes, hipMemcpyHostToDevice), "H2D copy");
+    LBM_HIP(transfer(const_cast<int32_t*>(src), s->staging, bytes, false, nullptr),
+            "H2D copy");
     LBM_HIP(launch_flags_set(s, b, (const int32_t*)s->staging, nullptr), "flags set kernel");
     LBM_HIP(hipStreamSynchronize(nullptr), "hipStreamSynchronize");
     return LBM_OK;
@@ -1212,14 +1212,22 @@ int state_copy(lbm_solver* s, void* host, uint64_t bytes, bool save)
     const size_t pitch = (size_t)s->stride * s->elem_bytes;
     char* h = (char*)host;
     char* d = (char*)s->dd;
-    if (save) {
-        LBM_HIP(hipMemcpy2D(h, plane, d, pitch, plane, kQ, hipMemcpyDeviceToHost), "D2H copy");
-        LBM_HIP(hipMemcpy(h + kQ * plane, s->flags, (size_t)s->n, hipMemcpyDeviceToHost),
-                "D2H copy");
+    const char* what = save ? "D2H copy" : "H2D copy";
+    if (ring_pays(host, bytes, kQ + 1)) {
+        Segment parts[kQ + 1];
+        for (int l = 0; l < kQ; l++)
+            parts[l] = Segment{h + l * plane, d + l * pitch, plane};
+        parts[kQ] = Segment{h + kQ * plane, s->flags, (size_t)s->n};
+        LBM_HIP(transfer(parts, kQ + 1, save, nullptr), what);
+        LBM_HIP(hipStreamSynchronize(nullptr), "hipStreamSynchronize");
+    } else if (save) {
+        LBM_HIP(hipMemcpy2D(h, plane, d, pitch, plane, kQ, hipMemcpyDeviceToHost), what);
+        LBM_HIP(hipMemcpy(h + kQ * plane, s->flags, (size_t)s->n, hipMemcpyDeviceToHost), what);
     } else {
-        LBM_HIP(hipMemcpy2D(d, pitch, h, plane, plane, kQ, hipMemcpyHostToDevice), "H2D copy");
-        LBM_HIP(hipMemcpy(s->flags, h + kQ * plane, (size_t)s->n, hipMemcpyHostToDevice),
-                "H2D copy");
+        LBM_HIP(hipMemcpy2D(d, pitch, h, plane, plane, kQ, hipMemcpyHostToDevice), what);
+        LBM_HIP(hipMemcpy(s->flags, h + kQ * plane, (size_t)s->n, hipMemcpyHostToDevice), what);
+    }
+    if (!save) {
         // a saved state was stored by the same formats, hence in range
         LBM_HIP(hipMemset(s->status, 0, sizeof(uint32_t)), "hipMemset");
         s->residual_valid = 0;

@@ -1,0 +1,255 @@
+// Copies between device memory and pageable host memory through a ring of
+// pinned buffers. The runtime's own copy into pageable memory moves 17 GB/s
+// (28 GB/s out of it): one thread, and the first touch of a fresh numpy array's
+// pages on top. PCIe moves 57 GB/s each way into pinned memory. Here the GPU
+// fills the ring while a few threads empty it into the destination (or the
+// reverse), page faults included: a 221 MB state saved into a new array in
+// 6 ms instead of 21, loaded in 5 instead of 8.
+#include <hip/hip_runtime.h>
+
+#include <atomic>
+#include <condition_variable>
+#include <cstring>
+#include <exception>
+#include <mutex>
+#include <thread>
+#include <vector>
+
+#include "lbm_transfer.hpp"
+
+namespace lbm {
+
+namespace {
+
+constexpr size_t kChunk = 8u << 20;
+constexpr size_t kSlots = 4;
+// below this the threads cost what they save; many small segments make many
+// small chunks (a 15 MB state of 20 parts 1.64 ms directly, 1.89 this way)
+constexpr size_t kLeast = 8u << 20, kLeastOfMany = 32u << 20;
+
+// The ring: 32 MiB for the process, taken with the first large transfer and
+// kept. One transfer uses it at a time; others meanwhile copy directly.
+std::mutex g_ring_mutex;
+char* g_ring = nullptr;
+
+bool take_ring()
+{
+    if (!g_ring) {
+        void* p = nullptr;
+        if (hipHostMalloc(&p, kSlots * kChunk, hipHostMallocPortable) != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        g_ring = (char*)p;
+    }
+    return true;
+}
+
+bool is_pinned(const void* p)
+{
+    hipPointerAttribute_t a;
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+        (void)hipGetLastError();   // pageable memory the runtime does not know
+        return false;
+    }
+    return a.type == hipMemoryTypeHost;
+}
+
+// Workers that copy their share of chunk 0, 1, ... between the ring and the
+// host, each chunk once the owner has let it go.
+class Workers {
+public:
+    Workers(const std::vector<Segment>& chunks, bool to_host) : chunks_(chunks), to_host_(to_host)
+    {
+        const unsigned hw = std::thread::hardware_concurrency();
+        count_ = hw < 4 ? 1 : hw < 16 ? hw / 2 : 8;
+    }
+    ~Workers() { stop(); }
+
+    // false when not a single thread could be started
+    bool start()
+    {
+        try {
+            for (unsigned t = 0; t < count_; t++)
+                threads_.emplace_back([this, t] { work(t); });
+        } catch (const std::exception&) {
+            stop();
+            return false;
+        }
+        return true;
+    }
+    // chunks [0, n) may be copied
+    void let(size_t n)
+    {
+        std::lock_guard<std::mutex> lock(m_);
+        if (n > let_)
+            let_ = n;
+        cv_work_.notify_all();
+    }
+    // until chunks [0, n) have been copied
+    void wait(size_t n)
+    {
+        std::unique_lock<std::mutex> lock(m_);
+        cv_done_.wait(lock, [&] { return done_ >= n; });
+    }
+    void stop()
+    {
+        {
+            std::lock_guard<std::mutex> lock(m_);
+            stop_ = true;
+            cv_work_.notify_all();
+        }
+        for (std::thread& t : threads_)
+            t.join();
+        threads_.clear();
+    }
+
+private:
+    void work(unsigned t)
+    {
+        for (size_t i = 0; i < chunks_.size(); i++) {
+            {
+                std::unique_lock<std::mutex> lock(m_);
+                cv_work_.wait(lock, [&] { return stop_ || let_ > i; });
+                if (stop_)
+                    return;
+            }
+            const Segment& c = chunks_[i];
+            const size_t lo = c.bytes * t / count_, hi = c.bytes * (t + 1) / count_;
+            char* slot = g_ring + (i % kSlots) * kChunk;
+            if (to_host_)
+                std::memcpy((char*)c.host + lo, slot + lo, hi - lo);
+            else
+                std::memcpy(slot + lo, (const char*)c.host + lo, hi - lo);
+            std::lock_guard<std::mutex> lock(m_);
+            // every worker passes the chunks in order: chunk i is done when
+            // the last of them has passed it
+            if (++passed_[i % kSlots] == count_) {
+                passed_[i % kSlots] = 0;
+                done_ = i + 1;
+                cv_done_.notify_all();
+            }
+        }
+    }
+
+    const std::vector<Segment>& chunks_;
+    const bool to_host_;
+    unsigned count_;
+    std::vector<std::thread> threads_;
+    std::mutex m_;
+    std::condition_variable cv_work_, cv_done_;
+    size_t let_ = 0, done_ = 0;
+    unsigned passed_[kSlots] = {};
+    bool stop_ = false;
+};
+
+struct Events {
+    hipEvent_t e[kSlots] = {};
+    ~Events()
+    {
+        for (hipEvent_t x : e)
+            if (x)
+                (void)hipEventDestroy(x);
+    }
+    hipError_t create()
+    {
+        for (hipEvent_t& x : e) {
+            const hipError_t r = hipEventCreateWithFlags(&x, hipEventDisableTiming);
+            if (r != hipSuccess)
+                return r;
+        }
+        return hipSuccess;
+    }
+};
+
+hipError_t direct(const Segment* segments, size_t count, bool to_host, hipStream_t st)
+{
+    for (size_t i = 0; i < count; i++) {
+        const Segment& s = segments[i];
+        const hipError_t e =
+            to_host ? hipMemcpyAsync(s.host, s.device, s.bytes, hipMemcpyDeviceToHost, st)
+                    : hipMemcpyAsync(s.device, s.host, s.bytes, hipMemcpyHostToDevice, st);
+        if (e != hipSuccess)
+            return e;
+    }
+    return to_host ? hipStreamSynchronize(st) : hipSuccess;
+}
+
+// The GPU's side of both directions. Slot i % kSlots holds chunk i: to the host
+// it is filled once the workers have emptied chunk i - kSlots and let go when
+// the copy into it has ended; to the device it is sent when the workers have
+// filled it and theirs again when that copy has ended.
+hipError_t through_ring(const std::vector<Segment>& chunks, bool to_host, hipStream_t st,
+                        Workers& w)
+{
+    Events ev;
+    hipError_t e = ev.create();
+    const size_t n = chunks.size();
+    if (!to_host)
+        w.let(n < kSlots ? n : kSlots);
+    for (size_t i = 0; e == hipSuccess && i < n; i++) {
+        const Segment& c = chunks[i];
+        char* slot = g_ring + (i % kSlots) * kChunk;
+        if (to_host) {
+            if (i >= kSlots)
+                w.wait(i - kSlots + 1);
+            e = hipMemcpyAsync(slot, c.device, c.bytes, hipMemcpyDeviceToHost, st);
+        } else {
+            w.wait(i + 1);
+            e = hipMemcpyAsync(c.device, slot, c.bytes, hipMemcpyHostToDevice, st);
+        }
+        if (e == hipSuccess)
+            e = hipEventRecord(ev.e[i % kSlots], st);
+        if (e == hipSuccess && i > 0) {   // one copy stays in flight
+            e = hipEventSynchronize(ev.e[(i - 1) % kSlots]);
+            if (e == hipSuccess)
+                w.let(to_host ? i : i - 1 + kSlots + 1);
+        }
+    }
+    if (e == hipSuccess)
+        e = hipStreamSynchronize(st);
+    if (e == hipSuccess && to_host) {
+        w.let(n);
+        w.wait(n);
+    }
+    return e;
+}
+
+}  // namespace
+
+bool ring_pays(const void* host, size_t bytes, size_t segments)
+{
+    return bytes >= (segments > 1 ? kLeastOfMany : kLeast) && !is_pinned(host);
+}
+
+hipError_t transfer(const Segment* segments, size_t count, bool to_host, hipStream_t st)
+{
+    size_t total = 0;
+    for (size_t i = 0; i < count; i++)
+        total += segments[i].bytes;
+    if (!ring_pays(segments[0].host, total, count))
+        return direct(segments, count, to_host, st);
+    std::unique_lock<std::mutex> ring(g_ring_mutex, std::try_to_lock);
+    if (!ring.owns_lock() || !take_ring())
+        return direct(segments, count, to_host, st);
+    std::vector<Segment> chunks;
+    try {
+        for (size_t i = 0; i < count; i++)
+            for (size_t at = 0; at < segments[i].bytes; at += kChunk) {
+                const size_t left = segments[i].bytes - at;
+                chunks.push_back({(char*)segments[i].host + at, (char*)segments[i].device + at,
+                                  left < kChunk ? left : kChunk});
+            }
+    } catch (const std::exception&) {
+        return direct(segments, count, to_host, st);
+    }
+    Workers w(chunks, to_host);
+    if (!w.start())
+        return direct(segments, count, to_host, st);
+    const hipError_t e = through_ring(chunks, to_host, st, w);
+    if (e != hipSuccess)
+        (void)hipStreamSynchronize(st);   // nothing reads or writes the ring any more
+    return e;
+}
+
+}  // namespace lbm
