@@ -267,13 +267,12 @@ inline uint64_t resident_bytes(const lbm_solver* s)
 //    alpha cached and uncapped, beta with one contiguous range of cells per
 //    XCD, whose L2 then serves the lines that neighbouring workgroups share:
 //    104^3 FP32 57.5 against 67-74, 140^3 129 against 147-150, FP64 112^3 134
-//    against 163, F16S 180^3 143 against 149. Level at 267 MB, 11 % slower at
-//    323 MB (three solvers in turn that need 254-258 MB together still gain).
+//    against 163. Level at 267 MB, 11 % slower at 323 MB (three solvers in turn
+//    that need 254-258 MB together still gain).
 //  * Only the state itself fits (a few steps, then another solver's turn): the
 //    XCD map loses (130^3 FP32 137-139 against 124-126), cached launches
 //    without it win, FP32 beta at 3 waves per SIMD (124.5 against 126.8 without
-//    a cap), 16-bit beta in 1024-thread workgroups (F16S 150^3 101 against
-//    105-110).
+//    a cap).
 //  * Otherwise the populations stream from HBM: FP32 / FP64 alpha nontemporal
 //    at 2 waves per SIMD. FP32 beta at 2 waves, in 256-thread workgroups with
 //    other solvers in between (200^3 469, other shapes 473-481); stepped alone
@@ -282,13 +281,20 @@ inline uint64_t resident_bytes(const lbm_solver* s)
 //    through LDS (300^3 1502 against 1514-1530, 512^3 7440 against 7585). FP64:
 //    to 400 MB the cached options still win (130^3 257 against 269-286), to
 //    800 MB beta at 2 waves (150^3 409 against 414), then through LDS (256^3
-//    1917 against 1956). F16S / BF16S beta in 1024-thread workgroups, one per
-//    CU (512^3 3970 against 4150 with two, 220^3 327 against 344), F16C, with
-//    more integer work per cell, two (512^3 4055 against 4285 in 256-thread
-//    ones); round robin over solvers that would each fit the cache 16-bit
-//    alpha nontemporal and beta with the XCD map (eight 130^3 F16S 729 against
-//    754-774).
+//    1917 against 1956).
+//  * The 16-bit formats beyond the L2s take two neighbouring cells per thread
+//    (4-byte accesses): F16S 130^3 57.9 against 59.5 for one cell per thread,
+//    61.6 against 65.3 with others in turn, 180^3 with others 157 against 161;
+//    streaming, where the caps of the FP32 steps pay now, 256^3 450 against
+//    505, 512^3 3800 against 3960, F16C 512^3 3850 against 4060, BF16S 400^3
+//    1769 against 1893, eight 130^3 F16S in turn 664 against 714. Within the L2s
+//    half the waves lose (62^3 13.2 against 12.4). Their rho / u stores would be
+//    every other word of two rows (300^3 F16C 986 against 955), so with outputs
+//    only the streaming alpha takes pairs and beta one cell per thread: 5 waves
+//    with the XCD map in the cache (130^3 65 without outputs), else 1024-thread
+//    workgroups (186 x 150 x 81 F16S 79 against 83-90, 400^3 2273 against 2329).
 constexpr int kCapWaves5 = 1 << 16;   // at most 5 waves per SIMD, 256-thread workgroups
+constexpr int kPairCells = 1 << 17;   // 16-bit formats: two neighbouring cells per thread
 
 inline int step_options(const lbm_solver* s, int kernel, uint64_t near, uint64_t far)
 {
@@ -300,22 +306,26 @@ inline int step_options(const lbm_solver* s, int kernel, uint64_t near, uint64_t
     far += own;
     const int p = s->p.precision;
     const bool half = p != LBM_F32 && p != LBM_F64;
+    if (half) {
+        const int pair = s->p.store_densities || s->p.store_velocities ? 0 : kPairCells;
+        if (near <= kCache && far <= 300 * MB)
+            return pair ? pair | (kernel == 0 ? 0 : LBM_LAUNCH_XCD_REMAP | LBM_LAUNCH_WAVES4)
+                        : (kernel == 0 ? 0 : LBM_LAUNCH_XCD_REMAP | kCapWaves5);
+        if (near <= kCache)
+            return pair ? pair | LBM_LAUNCH_WAVES4 : (kernel == 0 ? 0 : LBM_LAUNCH_BIG);
+        if (kernel == 0)
+            return kPairCells | LBM_LAUNCH_NONTEMPORAL | LBM_LAUNCH_WAVES3;
+        if (!pair)
+            return LBM_LAUNCH_BIG | LBM_LAUNCH_WAVES4;
+        return pair | (p == LBM_F16C ? LBM_LAUNCH_WAVES4 : LBM_LAUNCH_WAVES3) |
+               (own <= kCache ? LBM_LAUNCH_XCD_REMAP : 0);
+    }
     if (near <= kCache) {
         if (kernel == 0)
             return 0;
         if (far > 300 * MB)
-            return half ? LBM_LAUNCH_BIG : p == LBM_F32 ? LBM_LAUNCH_WAVES3 : 0;
-        return LBM_LAUNCH_XCD_REMAP | (p == LBM_F32   ? LBM_LAUNCH_WAVES2
-                                       : p == LBM_F64 ? LBM_LAUNCH_WAVES3
-                                                      : kCapWaves5);
-    }
-    if (half) {
-        if (own <= kCache)
-            return (kernel == 0 ? LBM_LAUNCH_NONTEMPORAL : LBM_LAUNCH_XCD_REMAP) |
-                   LBM_LAUNCH_WAVES4;
-        if (p == LBM_F16C)
-            return kernel == 0 ? 0 : LBM_LAUNCH_BIG;
-        return LBM_LAUNCH_WAVES4 | (kernel == 0 ? 0 : LBM_LAUNCH_BIG);
+            return p == LBM_F32 ? LBM_LAUNCH_WAVES3 : 0;
+        return LBM_LAUNCH_XCD_REMAP | (p == LBM_F32 ? LBM_LAUNCH_WAVES2 : LBM_LAUNCH_WAVES3);
     }
     if (p == LBM_F64 && own > kCache && own <= 400 * MB)
         return kernel == 0 ? 0 : LBM_LAUNCH_XCD_REMAP | LBM_LAUNCH_WAVES3;

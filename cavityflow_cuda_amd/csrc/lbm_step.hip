@@ -257,6 +257,110 @@ __global__ __launch_bounds__(kBlock) void k_beta_lds(StepArgs<typename P::C> a)
     }
 }
 
+// Two neighbouring cells per thread for the 16-bit formats: every access moves
+// both cells' codes of a plane in one 4-byte word (beta's planes start at any
+// even byte; unaligned words cost the memory nothing more than the shifted
+// halves did). A thread owns both cells' slots, so writing the codes of a cell
+// that stores nothing back beside its neighbour's changes nothing. The cells
+// take the per-cell code in turn, reading and writing their halves of the
+// words in registers.
+template <class S>
+struct AccHalf {
+    uint32_t* word;   // [19], registers
+    int high;
+    __device__ __forceinline__ AccHalf for_stores() const { return *this; }
+    __device__ __forceinline__ S load(int l, int32_t) const
+    {
+        return __builtin_bit_cast(S, (uint16_t)(high ? word[l] >> 16 : word[l]));
+    }
+    __device__ __forceinline__ void store(int l, int32_t, S v) const
+    {
+        const uint32_t c = __builtin_bit_cast(uint16_t, v);
+        word[l] = high ? (word[l] & 0xFFFFu) | (c << 16) : (word[l] & 0xFFFF0000u) | c;
+    }
+};
+
+using Word16 = uint32_t __attribute__((aligned(2)));
+
+template <bool NT>
+__device__ __forceinline__ uint32_t load_word(const char* base, uint32_t off)
+{
+    const LBM_GLOBAL Word16* p = (const LBM_GLOBAL Word16*)(base + off);
+    return NT ? __builtin_nontemporal_load(p) : *p;
+}
+template <bool NT>
+__device__ __forceinline__ void store_word(const char* base, uint32_t off, uint32_t v)
+{
+    LBM_GLOBAL Word16* p = (LBM_GLOBAL Word16*)(const_cast<char*>(base) + off);
+    if (NT)
+        __builtin_nontemporal_store(v, p);
+    else
+        *p = v;
+}
+
+template <class P, bool NT, int THREADS>
+__global__ __launch_bounds__(THREADS) void k_alpha_pair(StepArgs<typename P::C> a)
+{
+    using S = typename P::S;
+    const uint32_t blk = a.xcd ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x;
+    const uint32_t id = 2 * (blk * THREADS + threadIdx.x);
+    if (id + 1 >= a.cells) {
+        if (id < a.cells)
+            alpha_cell<P, kXfNone>(a, id, a.flags[id],
+                                   Acc32<S, NT>{a.plane, id * (uint32_t)sizeof(S)});
+        return;
+    }
+    uint32_t off = id * (uint32_t)sizeof(S);
+    uint32_t w[kQ];
+    const uint32_t flags = *(const uint16_t*)(a.flags + id);
+#pragma unroll
+    for (int l = 0; l < kQ; l++)
+        w[l] = load_word<NT>(a.plane[l], off);
+    const int f0 = flags & 255, f1 = flags >> 8;
+    alpha_cell<P, kXfNone>(a, id, f0, AccHalf<S>{w, 0});
+    alpha_cell<P, kXfNone>(a, id + 1, f1, AccHalf<S>{w, 1});
+    if (((f0 | f1) & (kFluid | kVelocityInjection)) == 0)
+        return;
+    off = fresh(off);
+#pragma unroll
+    for (int l = 0; l < kQ; l++)
+        store_word<NT>(a.plane[l], off, w[l]);
+}
+
+template <class P, bool NT, int THREADS>
+__global__ __launch_bounds__(THREADS) void k_beta_pair(StepArgs<typename P::C> a)
+{
+    using S = typename P::S;
+    const uint32_t blk = a.xcd ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x;
+    constexpr uint32_t kSpan = 2 * THREADS;
+    const uint32_t first = blk * kSpan, last = min(first + kSpan - 1, a.cells - 1);
+    const int64_t reach = (int64_t)a.nxy + a.nx + 1;
+    if ((int64_t)first < reach || (int64_t)last + reach >= (int64_t)a.n) {
+        // near the ends of the array: single cells, which wrap
+        for (uint32_t id = first + threadIdx.x; id <= last; id += THREADS) {
+            const AccWrap32<S> acc{(const char*)a.dd, a.stride, (int32_t)id, a.n};
+            beta_cell<P, kXfNone>(a, id, a.flags[id], acc);
+        }
+        return;
+    }
+    const uint32_t id = first + 2 * threadIdx.x;
+    uint32_t off = id * (uint32_t)sizeof(S);
+    uint32_t w[kQ];
+    const uint32_t flags = *(const uint16_t*)(a.flags + id);
+#pragma unroll
+    for (int l = 0; l < kQ; l++)
+        w[l] = load_word<NT>(a.plane[l], off);
+    const int f0 = flags & 255, f1 = flags >> 8;
+    beta_cell<P, kXfNone>(a, id, f0, AccHalf<S>{w, 0});
+    beta_cell<P, kXfNone>(a, id + 1, f1, AccHalf<S>{w, 1});
+    if (f0 == kObstacle && f1 == kObstacle)
+        return;
+    off = fresh(off);
+#pragma unroll
+    for (int l = 0; l < kQ; l++)
+        store_word<NT>(a.plane[l], off, w[l]);
+}
+
 // -------------------------------------------------------------- launches ---
 
 template <class P>
@@ -402,11 +506,45 @@ struct BetaK {
     static constexpr auto kernel = k_beta<P, FULL, OFF32, NT, SHAPE, XF>;
 };
 
+// kPairCells launches: BIG takes 1024-thread workgroups, the caps as for one
+// cell per thread. False when the step is not one of theirs.
+template <class P, int KERNEL>
+static bool launch_pair_cells(const lbm_solver* s, const Box& b, const StepArgs<typename P::C>& a,
+                              int opts, hipStream_t st)
+{
+    if constexpr (sizeof(typename P::S) == 2) {
+        if (!(opts & kPairCells) || !is_full(s, b) || !plane_off32(s) ||
+            (opts & LBM_LAUNCH_ADDR64) || face_work(s) != kXfNone)
+            return false;
+        const bool big = opts & LBM_LAUNCH_BIG, nt = opts & LBM_LAUNCH_NONTEMPORAL;
+        const bool any_cap = opts & (LBM_LAUNCH_WAVES2 | LBM_LAUNCH_WAVES3 | LBM_LAUNCH_WAVES4);
+        const size_t lds = big ? (any_cap ? kWideWaves2Lds : 0)
+                           : (opts & LBM_LAUNCH_WAVES2) ? kWaves2Lds
+                           : (opts & LBM_LAUNCH_WAVES3) ? kWaves3Lds
+                           : (opts & LBM_LAUNCH_WAVES4) ? kWaves4Lds
+                           : (opts & kCapWaves5)        ? kWaves5Lds : 0;
+        const uint32_t threads = big ? 1024 : 256, span = 2 * threads;
+        const dim3 grid((uint32_t)(((uint64_t)a.cells + span - 1) / span)), block(threads);
+        void (*kernel)(StepArgs<typename P::C>);
+        if (KERNEL == 0)
+            kernel = big ? (nt ? k_alpha_pair<P, true, 1024> : k_alpha_pair<P, false, 1024>)
+                         : (nt ? k_alpha_pair<P, true, 256> : k_alpha_pair<P, false, 256>);
+        else
+            kernel = big ? (nt ? k_beta_pair<P, true, 1024> : k_beta_pair<P, false, 1024>)
+                         : (nt ? k_beta_pair<P, true, 256> : k_beta_pair<P, false, 256>);
+        hipLaunchKernelGGL(kernel, grid, block, lds, st, a);
+        return true;
+    }
+    return false;
+}
+
 template <class P>
 static hipError_t alpha_t(const lbm_solver* s, const Box& b, int opts, hipStream_t st)
 {
     auto a = make_args<P>(s, b);
     a.xcd = (opts & LBM_LAUNCH_XCD_REMAP) ? 1 : 0;
+    if (launch_pair_cells<P, 0>(s, b, a, opts, st))
+        return hipGetLastError();
     if (is_full(s, b))
         launch_variant<P, AlphaK, true>(s, a, opts, st);
     else
@@ -451,6 +589,8 @@ static hipError_t beta_t(const lbm_solver* s, const Box& b, int opts, hipStream_
     for (int l = 0; l < kQ; l++)
         a.plane[l] += (int64_t)(cx(l) + cy(l) * a.nx + cz(l) * a.nxy) *
                       (int64_t)sizeof(typename P::S);
+    if (launch_pair_cells<P, 1>(s, b, a, opts, st))
+        return hipGetLastError();
     if ((opts & LBM_LAUNCH_LDS) && is_full(s, b) && plane_off32(s) && !(opts & LBM_LAUNCH_ADDR64)) {
         launch_beta_lds<P>(s, a, opts, st);
         return hipGetLastError();
