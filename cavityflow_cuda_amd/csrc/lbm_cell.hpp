@@ -58,8 +58,25 @@ __device__ __forceinline__ T fresh(T v)
     return v;
 }
 
+// outputs() stores a cell's rho and u where the solver keeps them.
+struct CellOutputs {
+    template <class C>
+    __device__ __forceinline__ void outputs(const StepArgs<C>& a, uint32_t id, C rho, C ux, C uy,
+                                            C uz) const
+    {
+        if (a.store_u) {
+            a.u[id] = ux;
+            a.u[a.stride + id] = uy;
+            a.u[2 * a.stride + id] = uz;
+        }
+        if (a.store_rho)
+            a.rho[id] = rho;
+    }
+};
+
 template <class S, bool NT>
-struct Acc32 {
+struct Acc32 : CellOutputs {
+    __device__ __forceinline__ Acc32(const char* const* p, uint32_t o) : plane(p), off(o) {}
     const char* const* plane;
     uint32_t off;
     __device__ __forceinline__ Acc32 for_stores() const { return {plane, fresh(off)}; }
@@ -89,7 +106,11 @@ __device__ __forceinline__ int32_t wrapped(int32_t id, int32_t delta, int32_t n)
 }
 
 template <class S>
-struct AccWrap32 {
+struct AccWrap32 : CellOutputs {
+    __device__ __forceinline__ AccWrap32(const char* d, int64_t st, int32_t i, int32_t cells)
+        : dd(d), stride(st), id(i), n(cells)
+    {
+    }
     const char* dd;
     int64_t stride;
     int32_t id, n;
@@ -107,7 +128,11 @@ struct AccWrap32 {
 };
 
 template <class S, bool WRAP>
-struct Acc64 {
+struct Acc64 : CellOutputs {
+    __device__ __forceinline__ Acc64(S* d, int64_t st, int32_t i, int32_t cells)
+        : dd(d), stride(st), id(i), n(cells)
+    {
+    }
     S* dd;
     int64_t stride;
     int32_t id, n;
@@ -458,13 +483,7 @@ __device__ __forceinline__ void alpha_cell(const StepArgs<typename P::C>& a, uin
         }
     }
 
-    if (a.store_u) {
-        a.u[id] = ux;
-        a.u[a.stride + id] = uy;
-        a.u[2 * a.stride + id] = uz;
-    }
-    if (a.store_rho)
-        a.rho[id] = rho;
+    acc.outputs(a, id, rho, ux, uy, uz);
 }
 
 
@@ -575,13 +594,7 @@ __device__ __forceinline__ void beta_cell(const StepArgs<typename P::C>& a, uint
     if (pack && kind != kStill)
         xpack_beta<P>(a, row, pl, pr, d);
 
-    if (a.store_u) {
-        a.u[id] = ux;
-        a.u[a.stride + id] = uy;
-        a.u[2 * a.stride + id] = uz;
-    }
-    if (a.store_rho)
-        a.rho[id] = rho;
+    acc.outputs(a, id, rho, ux, uy, uz);
 }
 
 

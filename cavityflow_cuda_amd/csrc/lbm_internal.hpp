@@ -283,18 +283,15 @@ inline uint64_t resident_bytes(const lbm_solver* s)
 //    800 MB beta at 2 waves (150^3 409 against 414), then through LDS (256^3
 //    1917 against 1956).
 //  * The 16-bit formats beyond the L2s take two neighbouring cells per thread
-//    (4-byte accesses): F16S 130^3 57.9 against 59.5 for one cell per thread,
-//    61.6 against 65.3 with others in turn, 180^3 with others 157 against 161;
+//    (4-byte accesses): F16S 130^3 57.7 against 59.7 for one cell per thread,
+//    61 against 64 with others in turn, 180^3 with others 157 against 161;
 //    streaming, where the caps of the FP32 steps pay now, 256^3 450 against
 //    505, 512^3 3800 against 3960, F16C 512^3 3850 against 4060, BF16S 400^3
-//    1769 against 1893, eight 130^3 F16S in turn 664 against 714. Within the L2s
-//    half the waves lose (62^3 13.2 against 12.4). Their rho / u stores would be
-//    every other word of two rows (300^3 F16C 986 against 955), so with outputs
-//    only the streaming alpha takes pairs and beta one cell per thread: 5 waves
-//    with the XCD map in the cache (130^3 65 without outputs), else 1024-thread
-//    workgroups (186 x 150 x 81 F16S 79 against 83-90, 400^3 2273 against 2329).
-constexpr int kCapWaves5 = 1 << 16;   // at most 5 waves per SIMD, 256-thread workgroups
-constexpr int kPairCells = 1 << 17;   // 16-bit formats: two neighbouring cells per thread
+//    1769 against 1893, eight 130^3 F16S in turn 664 against 714; with rho and
+//    u stored 186 x 150 x 81 69.0 against 70.6, 400^3 2256 against 2330 (256^3
+//    612 either way). Within the L2s half the waves lose (62^3 13.2 against
+//    12.4, 75^3 21.3 against 19.6).
+constexpr int kPairCells = 1 << 16;   // 16-bit formats: two neighbouring cells per thread
 
 inline int step_options(const lbm_solver* s, int kernel, uint64_t near, uint64_t far)
 {
@@ -307,17 +304,13 @@ inline int step_options(const lbm_solver* s, int kernel, uint64_t near, uint64_t
     const int p = s->p.precision;
     const bool half = p != LBM_F32 && p != LBM_F64;
     if (half) {
-        const int pair = s->p.store_densities || s->p.store_velocities ? 0 : kPairCells;
         if (near <= kCache && far <= 300 * MB)
-            return pair ? pair | (kernel == 0 ? 0 : LBM_LAUNCH_XCD_REMAP | LBM_LAUNCH_WAVES4)
-                        : (kernel == 0 ? 0 : LBM_LAUNCH_XCD_REMAP | kCapWaves5);
+            return kPairCells | (kernel == 0 ? 0 : LBM_LAUNCH_XCD_REMAP | LBM_LAUNCH_WAVES4);
         if (near <= kCache)
-            return pair ? pair | LBM_LAUNCH_WAVES4 : (kernel == 0 ? 0 : LBM_LAUNCH_BIG);
+            return kPairCells | LBM_LAUNCH_WAVES4;
         if (kernel == 0)
             return kPairCells | LBM_LAUNCH_NONTEMPORAL | LBM_LAUNCH_WAVES3;
-        if (!pair)
-            return LBM_LAUNCH_BIG | LBM_LAUNCH_WAVES4;
-        return pair | (p == LBM_F16C ? LBM_LAUNCH_WAVES4 : LBM_LAUNCH_WAVES3) |
+        return kPairCells | (p == LBM_F16C ? LBM_LAUNCH_WAVES4 : LBM_LAUNCH_WAVES3) |
                (own <= kCache ? LBM_LAUNCH_XCD_REMAP : 0);
     }
     if (near <= kCache) {

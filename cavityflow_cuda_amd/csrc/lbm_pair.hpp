@@ -105,7 +105,11 @@ struct PairLds {
 
 // Alpha of one window cell: inputs from registers, outputs to LDS.
 template <class S, int kWin>
-struct PairAlphaAcc {
+struct PairAlphaAcc : CellOutputs {
+    __device__ __forceinline__ PairAlphaAcc(const S* i, PairLds<S, kWin> m, int plane, int cell)
+        : in(i), lds(m), p(plane), c(cell)
+    {
+    }
     const S* in;  // the cell's 19 prefetched slots
     PairLds<S, kWin> lds;
     int p, c;
@@ -117,7 +121,12 @@ struct PairAlphaAcc {
 // Beta of one tile cell: inputs from LDS (slot l of the window cell c + c_l),
 // outputs to the destination buffer at id + c_l.
 template <class S, bool NTS, int kWin, int kWX>
-struct PairBetaAcc {
+struct PairBetaAcc : CellOutputs {
+    __device__ __forceinline__ PairBetaAcc(PairLds<S, kWin> m, int plane, int cell, S* d,
+                                           int64_t st, uint32_t i)
+        : lds(m), z(plane), c(cell), dst(d), stride(st), id(i)
+    {
+    }
     PairLds<S, kWin> lds;
     int z, c;
     S* dst;

@@ -188,7 +188,8 @@ __global__ __launch_bounds__(Shape<SHAPE>::kThreads) void k_beta(StepArgs<typena
 // lines' other cells. Blocks near the ends of the array (the linear wrap) and
 // box steps use the per-cell path.
 template <class S>
-struct AccLds {
+struct AccLds : CellOutputs {
+    __device__ __forceinline__ AccLds(S (*m)[kBlock], uint32_t i) : tile(m), t(i) {}
     S (*tile)[kBlock];
     uint32_t t;
     __device__ __forceinline__ AccLds for_stores() const { return *this; }
@@ -257,6 +258,13 @@ __global__ __launch_bounds__(kBlock) void k_beta_lds(StepArgs<typename P::C> a)
     }
 }
 
+// A cell's rho and u on their way to the pair's stores; GHOST_LAYER cells give
+// none in alpha.
+struct HalfOutputs {
+    float rho, u[3];
+    bool given = false;
+};
+
 // Two neighbouring cells per thread for the 16-bit formats: every access moves
 // both cells' codes of a plane in one 4-byte word (beta's planes start at any
 // even byte; unaligned words cost the memory nothing more than the shifted
@@ -264,10 +272,18 @@ __global__ __launch_bounds__(kBlock) void k_beta_lds(StepArgs<typename P::C> a)
 // that stores nothing back beside its neighbour's changes nothing. The cells
 // take the per-cell code in turn, reading and writing their halves of the
 // words in registers.
+// Bound by memory: F16S 512^3 moves its 20.8 GB of an alpha and a beta in
+// 3690 us, 5.6 TB/s (one cell per thread 4050 us).
 template <class S>
 struct AccHalf {
     uint32_t* word;   // [19], registers
+    HalfOutputs* out;
     int high;
+    __device__ __forceinline__ void outputs(const StepArgs<float>&, uint32_t, float rho, float ux,
+                                            float uy, float uz) const
+    {
+        *out = HalfOutputs{rho, {ux, uy, uz}, true};
+    }
     __device__ __forceinline__ AccHalf for_stores() const { return *this; }
     __device__ __forceinline__ S load(int l, int32_t) const
     {
@@ -298,12 +314,34 @@ __device__ __forceinline__ void store_word(const char* base, uint32_t off, uint3
         *p = v;
 }
 
-template <class P, bool NT, int THREADS>
-__global__ __launch_bounds__(THREADS) void k_alpha_pair(StepArgs<typename P::C> a)
+// Both cells' rho and u, 8 bytes at a time (id is even and the fields' planes
+// are multiples of 256 elements apart).
+__device__ __forceinline__ void store_outputs(const StepArgs<float>& a, uint32_t id,
+                                              const HalfOutputs (&o)[2])
+{
+    if (!a.store_u && !a.store_rho)
+        return;
+    if (o[0].given && o[1].given) {
+        if (a.store_u)
+#pragma unroll
+            for (int k = 0; k < 3; k++)
+                *(float2*)(a.u + k * a.stride + id) = make_float2(o[0].u[k], o[1].u[k]);
+        if (a.store_rho)
+            *(float2*)(a.rho + id) = make_float2(o[0].rho, o[1].rho);
+        return;
+    }
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+        if (o[h].given)
+            CellOutputs().outputs(a, id + h, o[h].rho, o[h].u[0], o[h].u[1], o[h].u[2]);
+}
+
+template <class P, bool NT>
+__global__ __launch_bounds__(kBlock) void k_alpha_pair(StepArgs<typename P::C> a)
 {
     using S = typename P::S;
     const uint32_t blk = a.xcd ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x;
-    const uint32_t id = 2 * (blk * THREADS + threadIdx.x);
+    const uint32_t id = 2 * (blk * kBlock + threadIdx.x);
     if (id + 1 >= a.cells) {
         if (id < a.cells)
             alpha_cell<P, kXfNone>(a, id, a.flags[id],
@@ -317,8 +355,10 @@ __global__ __launch_bounds__(THREADS) void k_alpha_pair(StepArgs<typename P::C> 
     for (int l = 0; l < kQ; l++)
         w[l] = load_word<NT>(a.plane[l], off);
     const int f0 = flags & 255, f1 = flags >> 8;
-    alpha_cell<P, kXfNone>(a, id, f0, AccHalf<S>{w, 0});
-    alpha_cell<P, kXfNone>(a, id + 1, f1, AccHalf<S>{w, 1});
+    HalfOutputs o[2];
+    alpha_cell<P, kXfNone>(a, id, f0, AccHalf<S>{w, &o[0], 0});
+    alpha_cell<P, kXfNone>(a, id + 1, f1, AccHalf<S>{w, &o[1], 1});
+    store_outputs(a, id, o);
     if (((f0 | f1) & (kFluid | kVelocityInjection)) == 0)
         return;
     off = fresh(off);
@@ -327,17 +367,17 @@ __global__ __launch_bounds__(THREADS) void k_alpha_pair(StepArgs<typename P::C> 
         store_word<NT>(a.plane[l], off, w[l]);
 }
 
-template <class P, bool NT, int THREADS>
-__global__ __launch_bounds__(THREADS) void k_beta_pair(StepArgs<typename P::C> a)
+template <class P>
+__global__ __launch_bounds__(kBlock) void k_beta_pair(StepArgs<typename P::C> a)
 {
     using S = typename P::S;
     const uint32_t blk = a.xcd ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x;
-    constexpr uint32_t kSpan = 2 * THREADS;
+    constexpr uint32_t kSpan = 2 * kBlock;
     const uint32_t first = blk * kSpan, last = min(first + kSpan - 1, a.cells - 1);
     const int64_t reach = (int64_t)a.nxy + a.nx + 1;
     if ((int64_t)first < reach || (int64_t)last + reach >= (int64_t)a.n) {
         // near the ends of the array: single cells, which wrap
-        for (uint32_t id = first + threadIdx.x; id <= last; id += THREADS) {
+        for (uint32_t id = first + threadIdx.x; id <= last; id += kBlock) {
             const AccWrap32<S> acc{(const char*)a.dd, a.stride, (int32_t)id, a.n};
             beta_cell<P, kXfNone>(a, id, a.flags[id], acc);
         }
@@ -349,16 +389,18 @@ __global__ __launch_bounds__(THREADS) void k_beta_pair(StepArgs<typename P::C> a
     const uint32_t flags = *(const uint16_t*)(a.flags + id);
 #pragma unroll
     for (int l = 0; l < kQ; l++)
-        w[l] = load_word<NT>(a.plane[l], off);
+        w[l] = load_word<false>(a.plane[l], off);
     const int f0 = flags & 255, f1 = flags >> 8;
-    beta_cell<P, kXfNone>(a, id, f0, AccHalf<S>{w, 0});
-    beta_cell<P, kXfNone>(a, id + 1, f1, AccHalf<S>{w, 1});
+    HalfOutputs o[2];
+    beta_cell<P, kXfNone>(a, id, f0, AccHalf<S>{w, &o[0], 0});
+    beta_cell<P, kXfNone>(a, id + 1, f1, AccHalf<S>{w, &o[1], 1});
+    store_outputs(a, id, o);
     if (f0 == kObstacle && f1 == kObstacle)
         return;
     off = fresh(off);
 #pragma unroll
     for (int l = 0; l < kQ; l++)
-        store_word<NT>(a.plane[l], off, w[l]);
+        store_word<false>(a.plane[l], off, w[l]);
 }
 
 // -------------------------------------------------------------- launches ---
@@ -428,7 +470,6 @@ static hipError_t init_t(const lbm_solver* s, hipStream_t st, int write_flags)
 // i.e. 4 (3, 2) waves per SIMD. Fewer resident waves means fewer concurrent
 // 19-plane streams, which the in-place FP32 steps turn into higher DRAM
 // efficiency.
-constexpr size_t kWaves5Lds = 27 * 1024 + 512;   // kCapWaves5
 constexpr size_t kWaves4Lds = 33 * 1024;
 constexpr size_t kWaves3Lds = 41 * 1024;
 constexpr size_t kWaves2Lds = 54 * 1024;
@@ -454,8 +495,7 @@ static void launch_shape(const lbm_solver* s, const StepArgs<typename P::C>& a, 
                                                                              : 0)
                        : (opts & LBM_LAUNCH_WAVES2) ? kWaves2Lds
                        : (opts & LBM_LAUNCH_WAVES3) ? kWaves3Lds
-                       : (opts & LBM_LAUNCH_WAVES4) ? kWaves4Lds
-                       : (opts & kCapWaves5)        ? kWaves5Lds : 0;
+                       : (opts & LBM_LAUNCH_WAVES4) ? kWaves4Lds : 0;
     const dim3 grid(blocks), block(G::kThreads);
     if (!plane_off32(s) || (opts & LBM_LAUNCH_ADDR64))
         hipLaunchKernelGGL((K<P, FULL, false, false, SHAPE, XF>::kernel), grid, block, lds, st, a);
@@ -506,33 +546,24 @@ struct BetaK {
     static constexpr auto kernel = k_beta<P, FULL, OFF32, NT, SHAPE, XF>;
 };
 
-// kPairCells launches: BIG takes 1024-thread workgroups, the caps as for one
-// cell per thread. False when the step is not one of theirs.
+// kPairCells launches, capped as one cell per thread is. False when the step is
+// not one of theirs.
 template <class P, int KERNEL>
 static bool launch_pair_cells(const lbm_solver* s, const Box& b, const StepArgs<typename P::C>& a,
                               int opts, hipStream_t st)
 {
     if constexpr (sizeof(typename P::S) == 2) {
-        if (!(opts & kPairCells) || !is_full(s, b) || !plane_off32(s) ||
-            (opts & LBM_LAUNCH_ADDR64) || face_work(s) != kXfNone)
+        if (!(opts & kPairCells) || !is_full(s, b) || !plane_off32(s) || face_work(s) != kXfNone)
             return false;
-        const bool big = opts & LBM_LAUNCH_BIG, nt = opts & LBM_LAUNCH_NONTEMPORAL;
-        const bool any_cap = opts & (LBM_LAUNCH_WAVES2 | LBM_LAUNCH_WAVES3 | LBM_LAUNCH_WAVES4);
-        const size_t lds = big ? (any_cap ? kWideWaves2Lds : 0)
-                           : (opts & LBM_LAUNCH_WAVES2) ? kWaves2Lds
-                           : (opts & LBM_LAUNCH_WAVES3) ? kWaves3Lds
-                           : (opts & LBM_LAUNCH_WAVES4) ? kWaves4Lds
-                           : (opts & kCapWaves5)        ? kWaves5Lds : 0;
-        const uint32_t threads = big ? 1024 : 256, span = 2 * threads;
-        const dim3 grid((uint32_t)(((uint64_t)a.cells + span - 1) / span)), block(threads);
-        void (*kernel)(StepArgs<typename P::C>);
-        if (KERNEL == 0)
-            kernel = big ? (nt ? k_alpha_pair<P, true, 1024> : k_alpha_pair<P, false, 1024>)
-                         : (nt ? k_alpha_pair<P, true, 256> : k_alpha_pair<P, false, 256>);
+        const size_t lds = (opts & LBM_LAUNCH_WAVES3)   ? kWaves3Lds
+                           : (opts & LBM_LAUNCH_WAVES4) ? kWaves4Lds : 0;
+        const dim3 grid((uint32_t)(((uint64_t)a.cells + 2 * kBlock - 1) / (2 * kBlock)));
+        if (KERNEL == 1)
+            hipLaunchKernelGGL(k_beta_pair<P>, grid, dim3(kBlock), lds, st, a);
+        else if (opts & LBM_LAUNCH_NONTEMPORAL)
+            hipLaunchKernelGGL((k_alpha_pair<P, true>), grid, dim3(kBlock), lds, st, a);
         else
-            kernel = big ? (nt ? k_beta_pair<P, true, 1024> : k_beta_pair<P, false, 1024>)
-                         : (nt ? k_beta_pair<P, true, 256> : k_beta_pair<P, false, 256>);
-        hipLaunchKernelGGL(kernel, grid, block, lds, st, a);
+            hipLaunchKernelGGL((k_alpha_pair<P, false>), grid, dim3(kBlock), lds, st, a);
         return true;
     }
     return false;
