@@ -316,7 +316,8 @@ class CavityController:
             return self._step_overlapped(1)
         if self.fused_x and not self._x_armed:
             raise RuntimeError("fused_x: the first step must be an alpha step")
-        for s in self.solvers.values():
+        # backwards: the subdomains alpha stepped last are still in the cache
+        for s in reversed(self.solvers.values()):
             s.simulationStepBeta(stream=self.stream)
         if not self.fused_x and len(self.solvers) > 1:
             self._exchange(1)

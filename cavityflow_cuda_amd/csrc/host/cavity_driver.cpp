@@ -240,12 +240,13 @@ public:
         const int phase = counter_ & 1;
         if (phase && !xrecv_.empty() && !xarmed_)
             throw lbm::Error(LBM_ERR_ARG, "--fused-x: the first step must be an alpha step");
-        for (auto& s : solvers_) {
-            if (phase)
-                s->simulationStepBeta();
-            else
+        // beta backwards: the subdomains alpha stepped last are still in the cache
+        if (phase)
+            for (size_t i = solvers_.size(); i-- > 0;)
+                solvers_[i]->simulationStepBeta();
+        else
+            for (auto& s : solvers_)
                 s->simulationStepAlpha();
-        }
         if (!xrecv_.empty()) {
             // from the first beta on: before it nothing was exchanged
             if (!xarmed_) {

@@ -240,12 +240,12 @@ int options_of_step(lbm_solver* s, int kernel, const Box& b)
     }
     __atomic_store_n(&s->step_mark, now, __ATOMIC_RELAXED);
     if (full || kernel != last)   // box steps of one half-step share its gap
-        __atomic_store_n(&s->step_gap, last < 0 ? 0 : gap, __ATOMIC_RELAXED);
+        __atomic_store_n(&s->step_gap, gap, __ATOMIC_RELAXED);
     if (!full || s->launch_set[kernel] || s->xpack[0] || s->xpack[1] || s->xunpack[0] ||
         s->xunpack[1] || !plane_off32(s))
         return s->launch[kernel];
-    if (last < 0)
-        return step_options(s, kernel, 0, 0);
+    if (last < 0)   // what others stepped since the solver was made
+        return step_options(s, kernel, gap, gap);
     return step_options(s, kernel, std::min(gap, gap_before), std::max(gap, gap_before));
 }
 
@@ -476,6 +476,7 @@ int lbm_create(const lbm_params* params, lbm_solver** out)
     s->launch[1] = default_launch(p.precision, 1, false, s->n >= kWideCells);
     s->launch_set[0] = s->launch_set[1] = 0;
     s->last_kernel = -1;
+    s->step_mark = g_stepped[s->p.device & 63].load(std::memory_order_relaxed);
     // round inv_tau / lid / gravity to the arithmetic type once
     if (p.precision != LBM_F64) {
         s->p.inv_tau = (float)p.inv_tau;

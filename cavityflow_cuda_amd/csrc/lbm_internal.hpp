@@ -58,6 +58,7 @@ struct StepArgs {
     C rest_rho;       // gravity_product, used when g is zero
     int store_rho, store_u;
     int xcd;          // renumber workgroups per XCD
+    int reverse;      // workgroups take the blocks of cells from the last to the first
     // byte address of plane l, shifted by the neighbour offset of direction l
     // for beta (0 for alpha): uniform per-plane bases for 32-bit lane offsets
     const char* plane[19];
@@ -255,11 +256,16 @@ inline uint64_t resident_bytes(const lbm_solver* s)
     return (uint64_t)s->n * (19 * s->elem_bytes + 1 + out * s->out_bytes);
 }
 
+// Internal launch options beside the LBM_LAUNCH_* ones.
+constexpr int kPairCells = 1 << 16;   // 16-bit formats: two neighbouring cells per thread
+constexpr int kReverse = 1 << 17;     // the last cells first
+
 // Launch options of a whole-domain step without face work whose kernel the
 // caller has not set. What decides is whether the state still lies in a cache
 // when the step starts: near and far are the lesser and the greater of the
 // bytes of other solvers stepped between this half-step and the solver's last,
-// and between that one and its predecessor. Times are us for an alpha and a beta.
+// and between that one and its predecessor. Times are us for an alpha and a
+// beta; "in turn": three solvers, one alpha and beta each.
 //  * Own bytes up to about the 8 L2s (4 MiB each): every workgroup is resident
 //    at once, no cap on the waves, no renumbering (62^3 FP32, 22 MB: 13.5
 //    against 15.9 with the streaming options; FP64 25.9 against 30.9).
@@ -267,71 +273,90 @@ inline uint64_t resident_bytes(const lbm_solver* s)
 //    alpha cached and uncapped, beta with one contiguous range of cells per
 //    XCD, whose L2 then serves the lines that neighbouring workgroups share:
 //    104^3 FP32 57.5 against 67-74, 140^3 129 against 147-150, FP64 112^3 134
-//    against 163. Level at 267 MB, 11 % slower at 323 MB (three solvers in turn
-//    that need 254-258 MB together still gain).
+//    against 163.
 //  * Only the state itself fits (a few steps, then another solver's turn): the
-//    XCD map loses (130^3 FP32 137-139 against 124-126), cached launches
-//    without it win, FP32 beta at 3 waves per SIMD (124.5 against 126.8 without
-//    a cap).
-//  * Otherwise the populations stream from HBM: FP32 / FP64 alpha nontemporal
-//    at 2 waves per SIMD. FP32 beta at 2 waves, in 256-thread workgroups with
-//    other solvers in between (200^3 469, other shapes 473-481); stepped alone
-//    up to 640 MB with the XCD map (160^3 222 against 232-238), then in
-//    1024-thread workgroups (220^3 587 against 600-605), and from 1.6 GB
-//    through LDS (300^3 1502 against 1514-1530, 512^3 7440 against 7585). FP64:
-//    to 400 MB the cached options still win (130^3 257 against 269-286), to
-//    800 MB beta at 2 waves (150^3 409 against 414), then through LDS (256^3
-//    1917 against 1956).
+//    XCD map loses for FP32 and FP64; beta in 1024-thread workgroups (FP32
+//    120^3 95.0 against 98.8 in 256-thread ones, 140^3 142.6 against 147.6),
+//    FP64 at 3 waves per SIMD (110^3 140.7 against 146.9); F16S with the map
+//    (150^3 88.0 against 93.1).
+//  * The state does not fit: beta takes the cells from the last to the first
+//    (kReverse), alpha from the first. Each then starts with what the other
+//    has just left in the Infinity Cache, up to 250 MB that need not come from
+//    HBM, as long as alpha stores them there (no nontemporal alpha). 185^3 FP32
+//    321 against 351, in turn 343 against 398; 229 x 186 x 141 with outputs
+//    337 / 352, 362 / 403; 256^3 905 / 934, 921 / 966; FP64 150^3 353 / 391,
+//    381 / 433, 192^3 780 / 809, 802 / 841, 256^3 1900 / 1944. Alpha at 2 waves
+//    per SIMD, with nothing else between and below 900 MB at 4 (175^3 275
+//    against 286). FP32 beta in 1024-thread workgroups, from 1.6 GB, where the
+//    saved part is small, through LDS with nontemporal alpha (512^3 7425
+//    against 7450 without the reversal, 400^3 3581 against 3603); FP64 through
+//    LDS from 1.8 GB, with nontemporal alpha from 3 GB.
+//  * Solvers that fit each but not together, stepped forwards by alpha and
+//    backwards by beta (the two gaps differ): the same, beta's range per XCD
+//    backwards; eight 82^3 FP32 322 against 344, eight 130^3 1147 against
+//    1174, four 162 x 82 x 82 FP64 494 against 521. Stepped round and round,
+//    nothing is left of them: nontemporal alpha, no reversal.
 //  * The 16-bit formats beyond the L2s take two neighbouring cells per thread
 //    (4-byte accesses): F16S 130^3 57.7 against 59.7 for one cell per thread,
-//    61 against 64 with others in turn, 180^3 with others 157 against 161;
-//    streaming, where the caps of the FP32 steps pay now, 256^3 450 against
-//    505, 512^3 3800 against 3960, F16C 512^3 3850 against 4060, BF16S 400^3
-//    1769 against 1893, eight 130^3 F16S in turn 664 against 714; with rho and
-//    u stored 186 x 150 x 81 69.0 against 70.6, 400^3 2256 against 2330 (256^3
-//    612 either way). Within the L2s half the waves lose (62^3 13.2 against
-//    12.4, 75^3 21.3 against 19.6).
-constexpr int kPairCells = 1 << 16;   // 16-bit formats: two neighbouring cells per thread
-
+//    61 against 64 with others in turn; streaming, 256^3 450 against 505,
+//    F16C 512^3 3850 against 4060, BF16S 400^3 1769 against 1893. Within the
+//    L2s half the waves lose (62^3 13.2 against 12.4). They gain less from the
+//    reversal: with rho and u stored (200^3 F16S in turn 282 against 302,
+//    300^3 906 against 978), above 1.2 GB (512^3 3747 against 3840) and in turn
+//    up to 800 MB (220^3 309 against 316); 200^3 alone loses (244 against 238).
 inline int step_options(const lbm_solver* s, int kernel, uint64_t near, uint64_t far)
 {
-    constexpr uint64_t MB = 1ull << 20, kL2 = 40 * MB, kCache = 260 * MB;
+    constexpr uint64_t MB = 1ull << 20, kL2 = 40 * MB, kCache = 250 * MB;
+    constexpr int NT = LBM_LAUNCH_NONTEMPORAL, XCD = LBM_LAUNCH_XCD_REMAP;
+    constexpr int W2 = LBM_LAUNCH_WAVES2, W3 = LBM_LAUNCH_WAVES3, W4 = LBM_LAUNCH_WAVES4;
+    constexpr int LDS = LBM_LAUNCH_LDS, BIG = LBM_LAUNCH_BIG, REV = kReverse;
     const uint64_t own = resident_bytes(s);
+    const int p = s->p.precision;
     if (own <= kL2)
         return 0;
     near += own;
     far += own;
-    const int p = s->p.precision;
-    const bool half = p != LBM_F32 && p != LBM_F64;
-    if (half) {
-        if (near <= kCache && far <= 300 * MB)
-            return kPairCells | (kernel == 0 ? 0 : LBM_LAUNCH_XCD_REMAP | LBM_LAUNCH_WAVES4);
+    const bool alone = far <= own + own / 4;      // no other solvers in between
+    const bool to_and_fro = far >= near + own / 2;
+    auto opts = [&](int alpha, int beta) { return kernel == 0 ? alpha : beta; };
+    if (p != LBM_F32 && p != LBM_F64) {
+        const bool wide_codes = p == LBM_F16C;    // more integer work per cell
+        const bool outputs = s->p.store_densities || s->p.store_velocities;
+        int o;
         if (near <= kCache)
-            return kPairCells | LBM_LAUNCH_WAVES4;
-        if (kernel == 0)
-            return kPairCells | LBM_LAUNCH_NONTEMPORAL | LBM_LAUNCH_WAVES3;
-        return kPairCells | (p == LBM_F16C ? LBM_LAUNCH_WAVES4 : LBM_LAUNCH_WAVES3) |
-               (own <= kCache ? LBM_LAUNCH_XCD_REMAP : 0);
+            o = far <= 300 * MB ? opts(0, XCD | W4) : wide_codes ? W4 : opts(W4, XCD | W3);
+        else if (own <= kCache)
+            o = opts(NT | W3, XCD | (wide_codes ? W4 : W3));
+        else if (own > 1200 * MB || (outputs && own > 800 * MB))
+            o = wide_codes ? opts(NT | W4, W4 | REV) : opts(NT | W3, W3 | REV);
+        else if (own > 800 * MB)
+            o = opts(NT | W3, wide_codes ? W4 : W3);
+        else if (outputs)
+            o = opts(W3, W3 | REV);
+        else if (alone || own <= 300 * MB)
+            o = own <= 500 * MB ? opts(NT | W4, W4) : opts(NT | W3, wide_codes ? W4 : W3);
+        else
+            o = opts(W3, W4 | REV);
+        return kPairCells | o;
     }
-    if (near <= kCache) {
-        if (kernel == 0)
-            return 0;
-        if (far > 300 * MB)
-            return p == LBM_F32 ? LBM_LAUNCH_WAVES3 : 0;
-        return LBM_LAUNCH_XCD_REMAP | (p == LBM_F32 ? LBM_LAUNCH_WAVES2 : LBM_LAUNCH_WAVES3);
+    if (near <= kCache && far <= 300 * MB)
+        return opts(0, XCD | (p == LBM_F32 ? W2 : W3));
+    if (near <= kCache)
+        return p == LBM_F32 ? opts(W3, BIG | W4) : opts(W2, W3);
+    if (own <= kCache) {
+        if (!to_and_fro)
+            return opts(NT | W2, W2);
+        const uint64_t all = (near + far) / 2;
+        return opts(p == LBM_F32 && all <= 600 * MB ? W3 : W2, XCD | W3 | REV);
     }
-    if (p == LBM_F64 && own > kCache && own <= 400 * MB)
-        return kernel == 0 ? 0 : LBM_LAUNCH_XCD_REMAP | LBM_LAUNCH_WAVES3;
-    if (kernel == 0)
-        return LBM_LAUNCH_NONTEMPORAL | LBM_LAUNCH_WAVES2;
-    if (p == LBM_F64)
-        return LBM_LAUNCH_WAVES2 | (own <= 800 * MB ? 0 : LBM_LAUNCH_LDS);
-    if (own >= 1600 * MB)
-        return LBM_LAUNCH_LDS | LBM_LAUNCH_WAVES4;
-    if (far > own + own / 4)   // other solvers in between
-        return LBM_LAUNCH_WAVES2;
-    return own < 640 * MB ? LBM_LAUNCH_XCD_REMAP | LBM_LAUNCH_WAVES3
-                          : LBM_LAUNCH_BIG | LBM_LAUNCH_WAVES4;
+    if (p == LBM_F32) {
+        if (own >= 1600 * MB)
+            return opts(NT | W2, LDS | W4 | REV);
+        return opts(alone && own <= 900 * MB ? W4 : own <= 300 * MB ? W3 : W2, BIG | W4 | REV);
+    }
+    if (own < 1800 * MB)
+        return opts(W2, (own <= 800 * MB ? W3 : W2) | REV);
+    return opts((own < 3000 * MB ? 0 : NT) | W2, LDS | W2 | REV);
 }
 
 // ||u - u_prev|| / ||u|| from the two FP64 sums; a non-finite state gives NaN

@@ -125,7 +125,7 @@ __global__ __launch_bounds__(Shape<SHAPE>::kThreads) void k_alpha(StepArgs<typen
 {
     using S = typename P::S;
     using G = Shape<SHAPE>;
-    const uint32_t blk = a.xcd ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x;
+    const uint32_t blk = step_block(a);
     for (uint32_t k = 0; k < G::kCells; k++) {
         const uint32_t gid = blk * G::kSpan + k * G::kThreads + threadIdx.x;
         if (gid >= a.cells)
@@ -146,7 +146,7 @@ __global__ __launch_bounds__(Shape<SHAPE>::kThreads) void k_beta(StepArgs<typena
 {
     using S = typename P::S;
     using G = Shape<SHAPE>;
-    const uint32_t blk = a.xcd ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x;
+    const uint32_t blk = step_block(a);
     // One decision per workgroup: neighbours of every cell of this block stay
     // inside [0, n) unless the block touches the first or last slab (box_cell
     // is increasing in gid, so the first and last cell bound the others).
@@ -202,7 +202,7 @@ __global__ __launch_bounds__(kBlock) void k_beta_lds(StepArgs<typename P::C> a)
 {
     using S = typename P::S;
     __shared__ S tile[kQ][kBlock];
-    const uint32_t blk = a.xcd ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x;
+    const uint32_t blk = step_block(a);
     const uint32_t b = blk * kBlock, t = threadIdx.x;
     const uint32_t last = min(b + kBlock - 1, a.cells - 1);
     const int64_t reach = (int64_t)a.nxy + a.nx + 1;
@@ -258,120 +258,19 @@ __global__ __launch_bounds__(kBlock) void k_beta_lds(StepArgs<typename P::C> a)
     }
 }
 
-// A cell's rho and u on their way to the pair's stores; GHOST_LAYER cells give
-// none in alpha.
-struct HalfOutputs {
-    float rho, u[3];
-    bool given = false;
-};
-
-// Two neighbouring cells per thread for the 16-bit formats: every access moves
-// both cells' codes of a plane in one 4-byte word (beta's planes start at any
-// even byte; unaligned words cost the memory nothing more than the shifted
-// halves did). A thread owns both cells' slots, so writing the codes of a cell
-// that stores nothing back beside its neighbour's changes nothing. The cells
-// take the per-cell code in turn, reading and writing their halves of the
-// words in registers.
-// Bound by memory: F16S 512^3 moves its 20.8 GB of an alpha and a beta in
-// 3690 us, 5.6 TB/s (one cell per thread 4050 us).
-template <class S>
-struct AccHalf {
-    uint32_t* word;   // [19], registers
-    HalfOutputs* out;
-    int high;
-    __device__ __forceinline__ void outputs(const StepArgs<float>&, uint32_t, float rho, float ux,
-                                            float uy, float uz) const
-    {
-        *out = HalfOutputs{rho, {ux, uy, uz}, true};
-    }
-    __device__ __forceinline__ AccHalf for_stores() const { return *this; }
-    __device__ __forceinline__ S load(int l, int32_t) const
-    {
-        return __builtin_bit_cast(S, (uint16_t)(high ? word[l] >> 16 : word[l]));
-    }
-    __device__ __forceinline__ void store(int l, int32_t, S v) const
-    {
-        const uint32_t c = __builtin_bit_cast(uint16_t, v);
-        word[l] = high ? (word[l] & 0xFFFFu) | (c << 16) : (word[l] & 0xFFFF0000u) | c;
-    }
-};
-
-using Word16 = uint32_t __attribute__((aligned(2)));
-
-template <bool NT>
-__device__ __forceinline__ uint32_t load_word(const char* base, uint32_t off)
-{
-    const LBM_GLOBAL Word16* p = (const LBM_GLOBAL Word16*)(base + off);
-    return NT ? __builtin_nontemporal_load(p) : *p;
-}
-template <bool NT>
-__device__ __forceinline__ void store_word(const char* base, uint32_t off, uint32_t v)
-{
-    LBM_GLOBAL Word16* p = (LBM_GLOBAL Word16*)(const_cast<char*>(base) + off);
-    if (NT)
-        __builtin_nontemporal_store(v, p);
-    else
-        *p = v;
-}
-
-// Both cells' rho and u, 8 bytes at a time (id is even and the fields' planes
-// are multiples of 256 elements apart).
-__device__ __forceinline__ void store_outputs(const StepArgs<float>& a, uint32_t id,
-                                              const HalfOutputs (&o)[2])
-{
-    if (!a.store_u && !a.store_rho)
-        return;
-    if (o[0].given && o[1].given) {
-        if (a.store_u)
-#pragma unroll
-            for (int k = 0; k < 3; k++)
-                *(float2*)(a.u + k * a.stride + id) = make_float2(o[0].u[k], o[1].u[k]);
-        if (a.store_rho)
-            *(float2*)(a.rho + id) = make_float2(o[0].rho, o[1].rho);
-        return;
-    }
-#pragma unroll
-    for (int h = 0; h < 2; h++)
-        if (o[h].given)
-            CellOutputs().outputs(a, id + h, o[h].rho, o[h].u[0], o[h].u[1], o[h].u[2]);
-}
-
+// Two cells per thread (lbm_cell.hpp) of one 16-bit domain.
 template <class P, bool NT>
 __global__ __launch_bounds__(kBlock) void k_alpha_pair(StepArgs<typename P::C> a)
 {
-    using S = typename P::S;
-    const uint32_t blk = a.xcd ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x;
-    const uint32_t id = 2 * (blk * kBlock + threadIdx.x);
-    if (id + 1 >= a.cells) {
-        if (id < a.cells)
-            alpha_cell<P, kXfNone>(a, id, a.flags[id],
-                                   Acc32<S, NT>{a.plane, id * (uint32_t)sizeof(S)});
-        return;
-    }
-    uint32_t off = id * (uint32_t)sizeof(S);
-    uint32_t w[kQ];
-    const uint32_t flags = *(const uint16_t*)(a.flags + id);
-#pragma unroll
-    for (int l = 0; l < kQ; l++)
-        w[l] = load_word<NT>(a.plane[l], off);
-    const int f0 = flags & 255, f1 = flags >> 8;
-    HalfOutputs o[2];
-    alpha_cell<P, kXfNone>(a, id, f0, AccHalf<S>{w, &o[0], 0});
-    alpha_cell<P, kXfNone>(a, id + 1, f1, AccHalf<S>{w, &o[1], 1});
-    store_outputs(a, id, o);
-    if (((f0 | f1) & (kFluid | kVelocityInjection)) == 0)
-        return;
-    off = fresh(off);
-#pragma unroll
-    for (int l = 0; l < kQ; l++)
-        store_word<NT>(a.plane[l], off, w[l]);
+    const uint32_t blk = step_block(a);
+    alpha_pair<P, NT>(a, 2 * (blk * kBlock + threadIdx.x));
 }
 
 template <class P>
 __global__ __launch_bounds__(kBlock) void k_beta_pair(StepArgs<typename P::C> a)
 {
     using S = typename P::S;
-    const uint32_t blk = a.xcd ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x;
+    const uint32_t blk = step_block(a);
     constexpr uint32_t kSpan = 2 * kBlock;
     const uint32_t first = blk * kSpan, last = min(first + kSpan - 1, a.cells - 1);
     const int64_t reach = (int64_t)a.nxy + a.nx + 1;
@@ -383,24 +282,7 @@ __global__ __launch_bounds__(kBlock) void k_beta_pair(StepArgs<typename P::C> a)
         }
         return;
     }
-    const uint32_t id = first + 2 * threadIdx.x;
-    uint32_t off = id * (uint32_t)sizeof(S);
-    uint32_t w[kQ];
-    const uint32_t flags = *(const uint16_t*)(a.flags + id);
-#pragma unroll
-    for (int l = 0; l < kQ; l++)
-        w[l] = load_word<false>(a.plane[l], off);
-    const int f0 = flags & 255, f1 = flags >> 8;
-    HalfOutputs o[2];
-    beta_cell<P, kXfNone>(a, id, f0, AccHalf<S>{w, &o[0], 0});
-    beta_cell<P, kXfNone>(a, id + 1, f1, AccHalf<S>{w, &o[1], 1});
-    store_outputs(a, id, o);
-    if (f0 == kObstacle && f1 == kObstacle)
-        return;
-    off = fresh(off);
-#pragma unroll
-    for (int l = 0; l < kQ; l++)
-        store_word<false>(a.plane[l], off, w[l]);
+    beta_pair<P>(a, first + 2 * threadIdx.x);
 }
 
 // -------------------------------------------------------------- launches ---
@@ -435,7 +317,7 @@ static StepArgs<typename P::C> make_args(const lbm_solver* s, const Box& b)
     a.rest_rho = gravity_product(a.g0, a.g1, a.g2);
     a.store_rho = s->p.store_densities;
     a.store_u = s->p.store_velocities;
-    a.xcd = 0;
+    a.xcd = a.reverse = 0;
     a.xpack[0] = (C*)s->xpack[0];
     a.xpack[1] = (C*)s->xpack[1];
     a.xunpack[0] = (const C*)s->xunpack[0];
@@ -574,6 +456,7 @@ static hipError_t alpha_t(const lbm_solver* s, const Box& b, int opts, hipStream
 {
     auto a = make_args<P>(s, b);
     a.xcd = (opts & LBM_LAUNCH_XCD_REMAP) ? 1 : 0;
+    a.reverse = (opts & kReverse) ? 1 : 0;
     if (launch_pair_cells<P, 0>(s, b, a, opts, st))
         return hipGetLastError();
     if (is_full(s, b))
@@ -616,6 +499,7 @@ static hipError_t beta_t(const lbm_solver* s, const Box& b, int opts, hipStream_
 {
     auto a = make_args<P>(s, b);
     a.xcd = (opts & LBM_LAUNCH_XCD_REMAP) ? 1 : 0;
+    a.reverse = (opts & kReverse) ? 1 : 0;
     // beta reads and writes plane l at id + c_l: fold the shift into the base
     for (int l = 0; l < kQ; l++)
         a.plane[l] += (int64_t)(cx(l) + cy(l) * a.nx + cz(l) * a.nxy) *
