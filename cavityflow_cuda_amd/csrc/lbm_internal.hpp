@@ -267,8 +267,14 @@ constexpr int kReverse = 1 << 17;     // the last cells first
 // and between that one and its predecessor. Times are us for an alpha and a
 // beta; "in turn": three solvers, one alpha and beta each.
 //  * Own bytes up to about the 8 L2s (4 MiB each): every workgroup is resident
-//    at once, no cap on the waves, no renumbering (62^3 FP32, 22 MB: 13.5
-//    against 15.9 with the streaming options; FP64 25.9 against 30.9).
+//    at once and no cap on the waves pays (62^3 FP32, 19 MB: 13.4 against 15.9
+//    with the streaming options). Both steps give each XCD the same contiguous
+//    range of cells, so that its L2 still holds them, and the z neighbours of
+//    beta, from one half-step to the next: 24 x 90 x 90 FP32 13.2 against 17.7
+//    without the map, 75^3 20.4 / 23.5, 50^3 FP64 16.3 / 21.3, 75^3 F16S 17.1 /
+//    20.3. Not below 2 MB (16^3 7.1 against 6.7), and not where a slab is a
+//    multiple of 8 workgroups, which places z neighbours on one XCD by itself
+//    (62^3 FP32 15.0 against 14.0; the other formats gain there too).
 //  * All within the 256 MB Infinity Cache (one cavity stepped again and again):
 //    alpha cached and uncapped, beta with one contiguous range of cells per
 //    XCD, whose L2 then serves the lines that neighbouring workgroups share:
@@ -312,8 +318,10 @@ inline int step_options(const lbm_solver* s, int kernel, uint64_t near, uint64_t
     constexpr int LDS = LBM_LAUNCH_LDS, BIG = LBM_LAUNCH_BIG, REV = kReverse;
     const uint64_t own = resident_bytes(s);
     const int p = s->p.precision;
-    if (own <= kL2)
-        return 0;
+    if (own <= kL2) {
+        const bool by_itself = p == LBM_F32 && s->size_h[0] * s->size_h[1] % (8 * 256) == 0;
+        return own <= 2 * MB || by_itself ? 0 : XCD;
+    }
     near += own;
     far += own;
     const bool alone = far <= own + own / 4;      // no other solvers in between
