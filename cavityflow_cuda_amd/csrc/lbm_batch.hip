@@ -74,10 +74,12 @@ __device__ __forceinline__ StepArgs<C> member_args(const MemberDesc& d, int phas
 // Tile iteration over [tile_lo, tile_hi): first tile and stride of this
 // workgroup (one tile, or a persistent stride over the range).
 __device__ __forceinline__ void tile_range(uint32_t tile_lo, uint32_t tile_hi, int persistent,
-                                           int xcd, uint32_t& first, uint32_t& step)
+                                           int order, uint32_t& first, uint32_t& step)
 {
     if (!persistent) {
-        first = tile_lo + (xcd ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x);
+        const uint32_t b = (order & LBM_LAUNCH_XCD_REMAP) ? xcd_block(blockIdx.x, gridDim.x)
+                                                          : blockIdx.x;
+        first = (order & kReverse) ? tile_hi - 1 - b : tile_lo + b;
         step = tile_hi;   // one tile only
     } else {
         first = tile_lo + blockIdx.x;
@@ -86,17 +88,18 @@ __device__ __forceinline__ void tile_range(uint32_t tile_lo, uint32_t tile_hi, i
 }
 
 // One kernel per phase (PHASE 0 = alpha, 1 = beta), so that each compiles to
-// the registers of its own half-step only.
-template <class P, int BLOCK, bool NT, int PHASE>
+// the registers of its own half-step only. PAIR: two neighbouring cells per
+// thread (16-bit formats, an even number of cells per thread).
+template <class P, int BLOCK, bool NT, int PHASE, bool PAIR>
 __global__ __launch_bounds__(BLOCK) void k_batch(const MemberDesc* __restrict__ mem,
                                                  const int32_t* __restrict__ tile_member,
                                                  uint32_t tile_lo, uint32_t tiles, int cpt,
-                                                 int persistent, int xcd)
+                                                 int persistent, int order)
 {
     using C = typename P::C;
     using S = typename P::S;
     uint32_t first, step;
-    tile_range(tile_lo, tiles, persistent, xcd, first, step);
+    tile_range(tile_lo, tiles, persistent, order, first, step);
     const uint32_t tile_cells = (uint32_t)BLOCK * (uint32_t)cpt;
     // A persistent workgroup strides over the tiles; consecutive tiles of a
     // large member share its descriptor, which is then read only once.
@@ -114,7 +117,17 @@ __global__ __launch_bounds__(BLOCK) void k_batch(const MemberDesc* __restrict__ 
             cur = m;
         }
         const uint32_t base = (t - tile_begin) * tile_cells;
-        if constexpr (PHASE == 0) {
+        const int64_t reach = (int64_t)a.nxy + a.nx + 1;
+        const int64_t last = std::min<int64_t>((int64_t)base + tile_cells, a.n) - 1;
+        const bool wrap = (int64_t)base < reach || last + reach >= (int64_t)a.n;
+        if constexpr (PHASE == 0 && PAIR) {
+            for (int k = 0; k < cpt; k += 2)
+                alpha_pair<P, NT>(a, base + (uint32_t)k * BLOCK + 2 * threadIdx.x);
+        } else if (PHASE == 1 && PAIR && !wrap) {
+            if constexpr (PHASE == 1 && PAIR)   // a tile that does not wrap is a whole one
+                for (int k = 0; k < cpt; k += 2)
+                    beta_pair<P>(a, base + (uint32_t)k * BLOCK + 2 * threadIdx.x);
+        } else if constexpr (PHASE == 0) {
             for (int k = 0; k < cpt; k++) {
                 const uint32_t id = base + (uint32_t)k * BLOCK + threadIdx.x;
                 if (id < (uint32_t)a.n) {
@@ -123,9 +136,6 @@ __global__ __launch_bounds__(BLOCK) void k_batch(const MemberDesc* __restrict__ 
                 }
             }
         } else {
-            const int64_t reach = (int64_t)a.nxy + a.nx + 1;
-            const int64_t last = std::min<int64_t>((int64_t)base + tile_cells, a.n) - 1;
-            const bool wrap = (int64_t)base < reach || last + reach >= (int64_t)a.n;
             for (int k = 0; k < cpt; k++) {
                 const uint32_t id = base + (uint32_t)k * BLOCK + threadIdx.x;
                 if (id >= (uint32_t)a.n)
@@ -172,6 +182,7 @@ struct lbm_batch {
     std::vector<Group> groups;
     uint64_t bytes = 0;        // of all members' populations
     bool tuned = false;        // the caller set (or autotuned) the tuning
+    int cpt = 1;               // cells per thread of the launches
     ResidualMember* res_mem = nullptr;   // members' residual inputs
     double* res_part = nullptr;          // members * kReduceBlocks * 5 partial sums
     double* res_out = nullptr;           // members * 5 sums
@@ -275,10 +286,25 @@ constexpr uint64_t kCacheGroup = 224ull << 20;
 
 static bool wide_storage(int precision) { return precision == LBM_F32 || precision == LBM_F64; }
 
-static int cached_options(int precision, int kernel)
+// All members within the L2s of the 8 XCDs: both half-steps give each XCD the
+// same tiles, which its L2 then still holds (6 cavities of 30 to 70 cells an
+// edge, 40 steps: FP32 411 us against 517 with the map for beta alone, F16S 357
+// against 408 to 533).
+static bool within_l2(const lbm_batch* b) { return b->bytes <= (40ull << 20); }
+
+// Neighbouring cells in pairs (alpha_pair, beta_pair): 12 cavities of 40 to 120
+// cells an edge, 40 steps, F16S 1.64 ms against 1.74, F16C 1.72 against 1.77; 20
+// of 48 to 128, 20 steps, 2.33 against 2.42 and 2.50 against 2.62. Within the
+// L2s half the waves lose (357 us against 374).
+static bool pairs_pay(const lbm_batch* b) { return !wide_storage(b->precision) && !within_l2(b); }
+
+static int cached_options(const lbm_batch* b, int kernel)
 {
-    return kernel == 0 ? 0
-                       : LBM_LAUNCH_XCD_REMAP | (wide_storage(precision) ? LBM_LAUNCH_WAVES4 : 0);
+    if (within_l2(b))
+        return LBM_LAUNCH_XCD_REMAP;
+    return kernel == 0
+               ? 0
+               : LBM_LAUNCH_XCD_REMAP | (wide_storage(b->precision) ? LBM_LAUNCH_WAVES4 : 0);
 }
 
 // The launch options of one half-step when `bytes` of members are stepped
@@ -288,9 +314,14 @@ static int options_of_tiles(const lbm_batch* b, uint64_t bytes, int kernel)
     if (b->tuned)
         return b->tuning.options[kernel];
     if (bytes <= kCacheGroup)
-        return cached_options(b->precision, kernel);
-    // streaming: nontemporal 16-bit alpha loses (29.0 against 24.7-26 ms above)
-    return wide_storage(b->precision) ? b->tuning.options[kernel] : 0;
+        return cached_options(b, kernel);
+    // streaming, beta from the last tile to the first: each half-step starts with
+    // what the other has left in the Infinity Cache (step_options)
+    if (!wide_storage(b->precision))
+        return kernel == 0 ? 0 : kReverse;   // nontemporal alpha loses (29.0, 24.7-26 ms above)
+    if (bytes <= (900ull << 20))
+        return kernel == 0 ? LBM_LAUNCH_WAVES4 : LBM_LAUNCH_WAVES4 | kReverse;
+    return b->tuning.options[kernel] | (kernel == 0 ? 0 : kReverse);
 }
 
 // Unused LDS reserved per workgroup for LBM_LAUNCH_WAVES4 / WAVES3 / WAVES2:
@@ -438,7 +469,12 @@ int apply_tuning(lbm_batch* b, const lbm_batch_tuning& t)
         free_alt(b);           // no pair pass: no second population buffers
     }
     b->tuning = t;
-    const uint32_t tile_cells = (uint32_t)(t.block * t.cells_per_thread);
+    b->bytes = 0;
+    for (const lbm_solver* s : b->members)
+        b->bytes += (uint64_t)kQ * s->stride * s->elem_bytes;
+    // no tuning set: one cell per thread, 16-bit formats beyond the L2s in pairs
+    b->cpt = b->tuned ? t.cells_per_thread : pairs_pay(b) ? 2 : 1;
+    const uint32_t tile_cells = (uint32_t)(t.block * b->cpt);
     int rc = upload_tiles(b, tile_cells, b->host_desc, &b->tile_member, &b->tiles, &b->desc);
     if (rc)
         return rc;
@@ -449,7 +485,6 @@ int apply_tuning(lbm_batch* b, const lbm_batch_tuning& t)
     const uint64_t cap = b->tuned ? (uint64_t)t.group_mb << 20 : kCacheGroup;
     uint64_t bytes = 0;
     uint32_t lo = 0, hi = 0;
-    b->bytes = 0;
     for (const lbm_solver* s : b->members) {
         const uint64_t mb = (uint64_t)kQ * s->stride * s->elem_bytes;
         const uint32_t mt = (uint32_t)((s->n + tile_cells - 1) / tile_cells);
@@ -460,7 +495,6 @@ int apply_tuning(lbm_batch* b, const lbm_batch_tuning& t)
         }
         hi += mt;
         bytes += mb;
-        b->bytes += mb;
     }
     b->groups.push_back({lo, hi, bytes});
     return LBM_OK;
@@ -503,30 +537,37 @@ hipError_t launch_pair(const lbm_batch* b, int parity, hipStream_t st)
     }
 }
 
-template <class P, int BLOCK>
-hipError_t launch_tiles_t(const lbm_batch* b, uint32_t lo, uint32_t hi, int phase, int opts,
+template <class P, int BLOCK, bool PAIR>
+hipError_t launch_tiles_c(const lbm_batch* b, uint32_t lo, uint32_t hi, int phase, int opts,
                           hipStream_t st)
 {
     const lbm_batch_tuning& t = b->tuning;
     const int persistent = t.waves_per_cu > 0;
     const uint32_t n = hi - lo;
     const uint32_t grid = persistent ? std::min<uint32_t>(n, (uint32_t)t.waves_per_cu * b->cus) : n;
-    const int xcd = (opts & LBM_LAUNCH_XCD_REMAP) ? 1 : 0;
+    const int order = opts & (LBM_LAUNCH_XCD_REMAP | kReverse);
     const size_t lds = waves_lds(opts, BLOCK);
     // nontemporal accesses only for alpha (beta's shifted pattern loses with them)
     if (phase != 0)
-        hipLaunchKernelGGL((k_batch<P, BLOCK, false, 1>), dim3(grid), dim3(BLOCK), lds, st,
-                           b->desc, b->tile_member, lo, hi, t.cells_per_thread, persistent,
-                           xcd);
+        hipLaunchKernelGGL((k_batch<P, BLOCK, false, 1, PAIR>), dim3(grid), dim3(BLOCK), lds,
+                           st, b->desc, b->tile_member, lo, hi, b->cpt, persistent, order);
     else if (opts & LBM_LAUNCH_NONTEMPORAL)
-        hipLaunchKernelGGL((k_batch<P, BLOCK, true, 0>), dim3(grid), dim3(BLOCK), lds, st,
-                           b->desc, b->tile_member, lo, hi, t.cells_per_thread, persistent,
-                           xcd);
+        hipLaunchKernelGGL((k_batch<P, BLOCK, true, 0, PAIR>), dim3(grid), dim3(BLOCK), lds,
+                           st, b->desc, b->tile_member, lo, hi, b->cpt, persistent, order);
     else
-        hipLaunchKernelGGL((k_batch<P, BLOCK, false, 0>), dim3(grid), dim3(BLOCK), lds, st,
-                           b->desc, b->tile_member, lo, hi, t.cells_per_thread, persistent,
-                           xcd);
+        hipLaunchKernelGGL((k_batch<P, BLOCK, false, 0, PAIR>), dim3(grid), dim3(BLOCK), lds,
+                           st, b->desc, b->tile_member, lo, hi, b->cpt, persistent, order);
     return hipGetLastError();
+}
+
+template <class P, int BLOCK>
+hipError_t launch_tiles_t(const lbm_batch* b, uint32_t lo, uint32_t hi, int phase, int opts,
+                          hipStream_t st)
+{
+    if constexpr (sizeof(typename P::S) == 2)
+        if (b->cpt % 2 == 0)
+            return launch_tiles_c<P, BLOCK, true>(b, lo, hi, phase, opts, st);
+    return launch_tiles_c<P, BLOCK, false>(b, lo, hi, phase, opts, st);
 }
 
 template <class P>
@@ -911,11 +952,11 @@ int lbm_batch_autotune(lbm_batch* b, int trial_steps, hipStream_t stream,
         // what a batch without a set tuning launches
         lbm_batch_tuning cand = start;
         cand.block = 256;
-        cand.cells_per_thread = 1;
+        cand.cells_per_thread = pairs_pay(b) ? 2 : 1;
         cand.waves_per_cu = 0;
         cand.group_mb = (int)(kCacheGroup >> 20);
         for (int ph = 0; ph < 2; ph++)
-            cand.options[ph] = cached_options(b->precision, ph);
+            cand.options[ph] = cached_options(b, ph);
         if ((rc = consider(cand)))
             return rc;
     }
