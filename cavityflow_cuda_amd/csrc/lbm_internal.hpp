@@ -178,7 +178,7 @@ hipError_t launch_residual_members(int precision, const ResidualMember* mem, int
                                    int layout, double* partials, double* out_dev,
                                    hipStream_t st);
 
-constexpr int kReduceBlocks = 2048;   // at most: 8 workgroups on each of 256 CUs
+constexpr int kReduceBlocks = 1024;   // at most: 4 workgroups on each of 256 CUs
 // Per-solver reduction buffer: kReduceBlocks * 5 partial sums, 5 results,
 // then the solver's overflow word (lbm_solver::status).
 constexpr size_t kPartialsBytes = (size_t)(kReduceBlocks + 1) * 5 * sizeof(double) + 64;

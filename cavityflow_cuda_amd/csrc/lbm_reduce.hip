@@ -20,7 +20,8 @@
 
 namespace lbm {
 
-constexpr int kRedBlock = 256;
+constexpr int kRedBlock = 512;       // 4 workgroups a CU, 8 waves per SIMD
+constexpr int kMomentsBlock = 256;
 constexpr int kRedVals = 5;
 
 __device__ __forceinline__ double wave_sum(double v)
@@ -235,12 +236,12 @@ __global__ __launch_bounds__(kRedBlock) void k_residual_members(const ResidualMe
 // Density and momentum of every cell of a box, computed from the populations
 // with the reference accumulation order; dst is dense [rho, jx, jy, jz][box].
 template <class P, int LAYOUT>
-__global__ __launch_bounds__(kRedBlock) void k_moments(const typename P::S* __restrict__ dd,
+__global__ __launch_bounds__(kMomentsBlock) void k_moments(const typename P::S* __restrict__ dd,
                                                        RedArgs a,
                                                        typename P::C* __restrict__ dst)
 {
     using C = typename P::C;
-    const uint32_t gid = blockIdx.x * kRedBlock + threadIdx.x;
+    const uint32_t gid = blockIdx.x * kMomentsBlock + threadIdx.x;
     if (gid >= a.cells)
         return;
     const uint32_t t = a.div_bx.div(gid);
@@ -378,12 +379,12 @@ static hipError_t moments_t(const lbm_solver* s, const Box& b, int layout, void*
                             hipStream_t st)
 {
     const RedArgs a = red_args(s, b);
-    const dim3 grid((a.cells + kRedBlock - 1) / kRedBlock);
+    const dim3 grid((a.cells + kMomentsBlock - 1) / kMomentsBlock);
     if (layout)
-        hipLaunchKernelGGL((k_moments<P, 1>), grid, dim3(kRedBlock), 0, st,
+        hipLaunchKernelGGL((k_moments<P, 1>), grid, dim3(kMomentsBlock), 0, st,
                            (const typename P::S*)s->dd, a, (typename P::C*)dst);
     else
-        hipLaunchKernelGGL((k_moments<P, 0>), grid, dim3(kRedBlock), 0, st,
+        hipLaunchKernelGGL((k_moments<P, 0>), grid, dim3(kMomentsBlock), 0, st,
                            (const typename P::S*)s->dd, a, (typename P::C*)dst);
     return hipGetLastError();
 }
@@ -449,7 +450,7 @@ hipError_t launch_residual_members(int precision, const ResidualMember* mem, int
 // ------------------------------------------------ allocation-free sums ---
 
 // Block partials of lbm_reduce_boxes_noalloc: LBM_NOALLOC_MAX_BOXES slices of
-// kReduceBlocks * kRedVals doubles (1.25 MiB). Every GPU the library runs on
+// kReduceBlocks * kRedVals doubles (640 KiB). Every GPU the library runs on
 // holds its own copy until the process ends. In host code `scratch` names a
 // host-side stand-in, not a device address, so it is never passed to a kernel
 // or a copy: each device's address comes from hipGetSymbolAddress, looked up

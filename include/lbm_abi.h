@@ -416,7 +416,7 @@ int lbm_reduce_box(lbm_solver* solver, const int origin[3], const int size[3], d
  * go to out_dev[5m..5m+4], caller-owned device memory, bit-identical to what
  * lbm_reduce_box returns for that solver and box. The block partials live in
  * a static device array of the library sized for LBM_NOALLOC_MAX_BOXES boxes
- * (1.25 MiB per GPU, held until the process ends); count outside
+ * (640 KiB per GPU, held until the process ends); count outside
  * 1..LBM_NOALLOC_MAX_BOXES is rejected with LBM_ERR_ARG. All solvers must
  * share one device and one precision. Asynchronous on `stream` (kernel
  * launches only: no allocation, copy or synchronisation). Calls that overlap
