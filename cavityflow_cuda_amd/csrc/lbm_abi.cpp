@@ -227,6 +227,12 @@ std::atomic<const lbm_solver*> g_last_stepped[64];
 int options_of_step(lbm_solver* s, int kernel, const Box& b)
 {
     const bool full = is_full(s, b);
+    // a tiny domain keeps its shape and puts nothing out of a cache: no account
+    if (resident_bytes(s) <= kTinyBytes)
+        return full && !s->launch_set[kernel] && !(s->xpack[0] || s->xpack[1] || s->xunpack[0] ||
+                                                   s->xunpack[1])
+                   ? 0
+                   : s->launch[kernel];
     const int dev = s->p.device & 63;
     uint64_t now = g_stepped[dev].load(std::memory_order_relaxed);
     // relaxed atomics: threads that step boxes of one solver side by side may
@@ -435,8 +441,8 @@ int lbm_device_bytes(const lbm_params* params, int pair_buffer, uint64_t* bytes)
     int rc = check_params(*params, "lbm_device_bytes", &n);
     if (rc)
         return rc;
-    const uint64_t stride = (uint64_t)(n + 255) / 256 * 256;
     const uint64_t eb = (uint64_t)element_bytes(params->precision);
+    const uint64_t stride = (uint64_t)(n + 255) / 256 * 256;
     const uint64_t ob = params->precision == LBM_F64 ? 8 : 4;
     uint64_t b = (uint64_t)kQ * stride * eb + stride;                  // populations, flags
     b += params->store_densities ? stride * ob : 0;

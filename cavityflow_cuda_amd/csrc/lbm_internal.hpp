@@ -256,6 +256,8 @@ inline uint64_t resident_bytes(const lbm_solver* s)
     return (uint64_t)s->n * (19 * s->elem_bytes + 1 + out * s->out_bytes);
 }
 
+constexpr uint64_t kTinyBytes = 2ull << 20;   // see step_options
+
 // Internal launch options beside the LBM_LAUNCH_* ones.
 constexpr int kPairCells = 1 << 16;   // 16-bit formats: two neighbouring cells per thread
 constexpr int kReverse = 1 << 17;     // the last cells first
@@ -320,7 +322,7 @@ inline int step_options(const lbm_solver* s, int kernel, uint64_t near, uint64_t
     const int p = s->p.precision;
     if (own <= kL2) {
         const bool by_itself = p == LBM_F32 && s->size_h[0] * s->size_h[1] % (8 * 256) == 0;
-        return own <= 2 * MB || by_itself ? 0 : XCD;
+        return own <= kTinyBytes || by_itself ? 0 : XCD;
     }
     near += own;
     far += own;
