@@ -251,7 +251,7 @@ int options_of_step(lbm_solver* s, int kernel, const Box& b)
         s->xunpack[1] || !plane_off32(s))
         return s->launch[kernel];
     if (last < 0)   // what others stepped since the solver was made
-        return step_options(s, kernel, gap, gap);
+        return step_options(s, kernel, gap, gap, true);
     return step_options(s, kernel, std::min(gap, gap_before), std::max(gap, gap_before));
 }
 

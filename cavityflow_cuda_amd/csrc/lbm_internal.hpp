@@ -299,6 +299,9 @@ constexpr int kReverse = 1 << 17;     // the last cells first
 //    saved part is small, through LDS with nontemporal alpha (512^3 7425
 //    against 7450 without the reversal, 400^3 3581 against 3603); FP64 through
 //    LDS from 1.8 GB, with nontemporal alpha from 3 GB.
+//    The very first alpha of a solver (`first`) stays nontemporal up to there: the
+//    caches still hold part of what its creation wrote, which a cached alpha
+//    would put out (229 x 186 x 141 383 against 391, 192^3 FP64 852 against 866).
 //  * Solvers that fit each but not together, stepped forwards by alpha and
 //    backwards by beta (the two gaps differ): the same, beta's range per XCD
 //    backwards; eight 82^3 FP32 322 against 344, eight 130^3 1147 against
@@ -312,7 +315,8 @@ constexpr int kReverse = 1 << 17;     // the last cells first
 //    reversal: with rho and u stored (200^3 F16S in turn 282 against 302,
 //    300^3 906 against 978), above 1.2 GB (512^3 3747 against 3840) and in turn
 //    up to 800 MB (220^3 309 against 316); 200^3 alone loses (244 against 238).
-inline int step_options(const lbm_solver* s, int kernel, uint64_t near, uint64_t far)
+inline int step_options(const lbm_solver* s, int kernel, uint64_t near, uint64_t far,
+                        bool first = false)
 {
     constexpr uint64_t MB = 1ull << 20, kL2 = 40 * MB, kCache = 250 * MB;
     constexpr int NT = LBM_LAUNCH_NONTEMPORAL, XCD = LBM_LAUNCH_XCD_REMAP;
@@ -353,6 +357,8 @@ inline int step_options(const lbm_solver* s, int kernel, uint64_t near, uint64_t
         return opts(0, XCD | (p == LBM_F32 ? W2 : W3));
     if (near <= kCache)
         return p == LBM_F32 ? opts(W3, BIG | W4) : opts(W2, W3);
+    if (first && kernel == 0 && own < 1600 * MB)
+        return NT | W2;
     if (own <= kCache) {
         if (!to_and_fro)
             return opts(NT | W2, W2);
