@@ -34,7 +34,7 @@ struct MemberDesc {
     int64_t stride;
     int32_t n, nx, nxy;
     uint32_t tile_begin;
-    int32_t store_rho, store_u;
+    int32_t store_rho, store_u, store_walls;
     double inv_tau, lid, g0, g1, g2, rest_rho;
     int32_t gravity;
     uint32_t* status;
@@ -61,6 +61,7 @@ __device__ __forceinline__ StepArgs<C> member_args(const MemberDesc& d, int phas
     a.rest_rho = (C)d.rest_rho;
     a.store_rho = d.store_rho;
     a.store_u = d.store_u;
+    a.store_walls = d.store_walls;
     a.xpack_on = 0;
     a.xpack[0] = a.xpack[1] = nullptr;
     a.xunpack[0] = a.xunpack[1] = nullptr;
@@ -700,6 +701,7 @@ int lbm_batch_create(lbm_solver* const* members, int count, lbm_batch** out)
         d.nxy = nxy;
         d.store_rho = s->p.store_densities;
         d.store_u = s->p.store_velocities;
+        d.store_walls = is_closed(s);
         d.inv_tau = s->p.inv_tau;
         d.lid = s->p.lid_velocity;
         d.g0 = s->p.gravitation[0];

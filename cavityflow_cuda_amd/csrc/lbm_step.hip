@@ -317,6 +317,7 @@ static StepArgs<typename P::C> make_args(const lbm_solver* s, const Box& b)
     a.rest_rho = gravity_product(a.g0, a.g1, a.g2);
     a.store_rho = s->p.store_densities;
     a.store_u = s->p.store_velocities;
+    a.store_walls = is_closed(s);
     a.xcd = a.reverse = 0;
     a.xpack[0] = (C*)s->xpack[0];
     a.xpack[1] = (C*)s->xpack[1];

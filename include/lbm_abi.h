@@ -172,6 +172,13 @@ int lbm_simulation_step_alpha(lbm_solver* solver, const int origin[3], const int
 int lbm_simulation_step_beta(lbm_solver* solver, const int origin[3], const int size[3],
                              hipStream_t stream);
 
+/* What a step leaves alone: alpha stores no population of a GHOST_LAYER cell, and
+ * neither step one of an OBSTACLE cell (in beta: the slots it reads), so that a
+ * face transfer on another stream may fill them meanwhile. Except: the
+ * whole-domain steps of 16-bit solvers, alone or in a batch, that were created
+ * without a GHOST_LAYER face may store those of an OBSTACLE cell back as they
+ * read them. */
+
 /* Launch variants of the step kernels; they change speed, never results.
  * kernel: 0 = alpha, 1 = beta. Options set here are the ones every launch of
  * that kernel takes. Whole-domain steps of a kernel that was not set, without
