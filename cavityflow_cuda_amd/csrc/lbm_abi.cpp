@@ -238,8 +238,9 @@ int options_of_step(lbm_solver* s, int kernel, const Box& b)
     // relaxed atomics: threads that step boxes of one solver side by side may
     // both write the marks
     const uint64_t gap = now - __atomic_load_n(&s->step_mark, __ATOMIC_RELAXED);
-    const uint64_t gap_before = __atomic_load_n(&s->step_gap, __ATOMIC_RELAXED);
     const int last = __atomic_exchange_n(&s->last_kernel, kernel, __ATOMIC_RELAXED);
+    // no half-step yet: what others stepped since the solver was made
+    const uint64_t gap_before = last < 0 ? gap : __atomic_load_n(&s->step_gap, __ATOMIC_RELAXED);
     if (g_last_stepped[dev].exchange(s, std::memory_order_relaxed) != s) {
         const uint64_t bytes = resident_bytes(s);
         now = g_stepped[dev].fetch_add(bytes, std::memory_order_relaxed) + bytes;
@@ -250,8 +251,6 @@ int options_of_step(lbm_solver* s, int kernel, const Box& b)
     if (!full || s->launch_set[kernel] || s->xpack[0] || s->xpack[1] || s->xunpack[0] ||
         s->xunpack[1] || !plane_off32(s))
         return s->launch[kernel];
-    if (last < 0)   // what others stepped since the solver was made
-        return step_options(s, kernel, gap, gap, true);
     return step_options(s, kernel, std::min(gap, gap_before), std::max(gap, gap_before));
 }
 

@@ -312,9 +312,6 @@ constexpr int kReverse = 1 << 17;     // the last cells first
 //    saved part is small, through LDS with nontemporal alpha (512^3 7425
 //    against 7450 without the reversal, 400^3 3581 against 3603); FP64 through
 //    LDS from 1.8 GB, with nontemporal alpha from 3 GB.
-//    The very first alpha of a solver (`first`) stays nontemporal up to there: the
-//    caches still hold part of what its creation wrote, which a cached alpha
-//    would put out (229 x 186 x 141 383 against 391, 192^3 FP64 852 against 866).
 //  * Solvers that fit each but not together, stepped forwards by alpha and
 //    backwards by beta (the two gaps differ): the same, beta's range per XCD
 //    backwards; eight 82^3 FP32 322 against 344, eight 130^3 1147 against
@@ -331,8 +328,7 @@ constexpr int kReverse = 1 << 17;     // the last cells first
 //    Domains with GHOST_LAYER faces store half words at their walls and ghosts,
 //    which nontemporal neighbours in the line turn into reads of the memory:
 //    always cached (250^3 462 against 519, 400^3 1890 / 2130).
-inline int step_options(const lbm_solver* s, int kernel, uint64_t near, uint64_t far,
-                        bool first = false)
+inline int step_options(const lbm_solver* s, int kernel, uint64_t near, uint64_t far)
 {
     constexpr uint64_t MB = 1ull << 20, kL2 = 40 * MB, kCache = 250 * MB;
     constexpr int NT = LBM_LAUNCH_NONTEMPORAL, XCD = LBM_LAUNCH_XCD_REMAP;
@@ -373,8 +369,6 @@ inline int step_options(const lbm_solver* s, int kernel, uint64_t near, uint64_t
         return opts(0, XCD | (p == LBM_F32 ? W2 : W3));
     if (near <= kCache)
         return p == LBM_F32 ? opts(W3, BIG | W4) : opts(W2, W3);
-    if (first && kernel == 0 && own < 1600 * MB)
-        return NT | W2;
     if (own <= kCache) {
         if (!to_and_fro)
             return opts(NT | W2, W2);
