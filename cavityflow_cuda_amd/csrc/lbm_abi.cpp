@@ -213,12 +213,35 @@ int copy_set(lbm_solver* s, int field, const Box& b, int ncomp, const void* src,
     return LBM_OK;
 }
 
-// Bytes of domains stepped so far on each device (modulo the arrays), several
-// half-steps of one solver in a row counted once: what passed between two
-// half-steps of a solver says whether its state can still be in the caches.
-// Only launch shapes depend on it, never results.
+// Bytes of domains stepped, or written as a whole, so far on each device (modulo
+// the arrays), several in a row of one solver counted once: what passed between
+// two half-steps of a solver says whether its state can still be in the caches.
+// Only launch shapes depend on it, never results. Relaxed atomics: threads that
+// step boxes of one solver side by side may both write the marks.
 std::atomic<uint64_t> g_stepped[64];
 std::atomic<const lbm_solver*> g_last_stepped[64];
+
+void count_passed(lbm_solver* s)
+{
+    const int dev = s->p.device & 63;
+    const uint64_t bytes = resident_bytes(s);
+    const uint64_t now =
+        g_last_stepped[dev].exchange(s, std::memory_order_relaxed) != s
+            ? g_stepped[dev].fetch_add(bytes, std::memory_order_relaxed) + bytes
+            : g_stepped[dev].load(std::memory_order_relaxed);
+    __atomic_store_n(&s->step_mark, now, __ATOMIC_RELAXED);
+}
+
+// Every cell was created, reset, loaded or set: the next half-step's gap counts
+// from here.
+void count_written(lbm_solver* s)
+{
+    if (resident_bytes(s) <= kTinyBytes)
+        return;
+    count_passed(s);
+    __atomic_store_n(&s->last_kernel, -1, __ATOMIC_RELAXED);
+    __atomic_store_n(&s->streamed, 0, __ATOMIC_RELAXED);
+}
 
 // The launch options of a step: the ones set (or the defaults by face work and
 // size), and for whole-domain steps without face work of a kernel the caller
@@ -233,25 +256,23 @@ int options_of_step(lbm_solver* s, int kernel, const Box& b)
                                                    s->xunpack[1])
                    ? 0
                    : s->launch[kernel];
-    const int dev = s->p.device & 63;
-    uint64_t now = g_stepped[dev].load(std::memory_order_relaxed);
-    // relaxed atomics: threads that step boxes of one solver side by side may
-    // both write the marks
+    const uint64_t now = g_stepped[s->p.device & 63].load(std::memory_order_relaxed);
     const uint64_t gap = now - __atomic_load_n(&s->step_mark, __ATOMIC_RELAXED);
     const int last = __atomic_exchange_n(&s->last_kernel, kernel, __ATOMIC_RELAXED);
-    // no half-step yet: what others stepped since the solver was made
+    // no half-step since the state was written
     const uint64_t gap_before = last < 0 ? gap : __atomic_load_n(&s->step_gap, __ATOMIC_RELAXED);
-    if (g_last_stepped[dev].exchange(s, std::memory_order_relaxed) != s) {
-        const uint64_t bytes = resident_bytes(s);
-        now = g_stepped[dev].fetch_add(bytes, std::memory_order_relaxed) + bytes;
-    }
-    __atomic_store_n(&s->step_mark, now, __ATOMIC_RELAXED);
+    count_passed(s);
     if (full || kernel != last)   // box steps of one half-step share its gap
         __atomic_store_n(&s->step_gap, gap, __ATOMIC_RELAXED);
-    if (!full || s->launch_set[kernel] || s->xpack[0] || s->xpack[1] || s->xunpack[0] ||
-        s->xunpack[1] || !plane_off32(s))
-        return s->launch[kernel];
-    return step_options(s, kernel, std::min(gap, gap_before), std::max(gap, gap_before));
+    const bool chosen = full && !s->launch_set[kernel] && !s->xpack[0] && !s->xpack[1] &&
+                        !s->xunpack[0] && !s->xunpack[1] && plane_off32(s);
+    const int options =
+        chosen ? step_options(s, kernel, std::min(gap, gap_before), std::max(gap, gap_before),
+                              __atomic_load_n(&s->streamed, __ATOMIC_RELAXED) != 0)
+               : s->launch[kernel];
+    __atomic_store_n(&s->streamed, kernel == 0 && (options & LBM_LAUNCH_NONTEMPORAL) ? 1 : 0,
+                     __ATOMIC_RELAXED);
+    return options;
 }
 
 // norm . c_l > 0 mask of setDensityDistributions(..., direction, ...)
@@ -493,8 +514,6 @@ int lbm_create(const lbm_params* params, lbm_solver** out)
     s->launch[0] = default_launch(p.precision, 0, false, s->n >= kWideCells);
     s->launch[1] = default_launch(p.precision, 1, false, s->n >= kWideCells);
     s->launch_set[0] = s->launch_set[1] = 0;
-    s->last_kernel = -1;
-    s->step_mark = g_stepped[s->p.device & 63].load(std::memory_order_relaxed);
     // round inv_tau / lid / gravity to the arithmetic type once
     if (p.precision != LBM_F64) {
         s->p.inv_tau = (float)p.inv_tau;
@@ -534,6 +553,8 @@ int lbm_create(const lbm_params* params, lbm_solver** out)
         lbm_destroy(s);
         return LBM_ERR_HIP;
     }
+    s->last_kernel = -1;
+    count_written(s);
     *out = s;
     return LBM_OK;
 }
@@ -655,6 +676,8 @@ int lbm_set_density_distributions(lbm_solver* s, const int origin[3], const int 
     }
     if ((rc = set_device(s)))
         return rc;
+    if (b.bx >= s->p.size[0] && b.by >= s->p.size[1] && b.bz >= s->p.size[2])
+        count_written(s);
     return copy_set(s, 0, b, kQ, src, src_on_device, 0x7FFFFu, stream);
 }
 
@@ -1199,6 +1222,7 @@ int lbm_reset(lbm_solver* s)
     LBM_HIP(launch_init(s, nullptr, 0), "init kernel");
     LBM_HIP(hipStreamSynchronize(nullptr), "hipStreamSynchronize");
     s->residual_valid = 0;
+    count_written(s);
     return LBM_OK;
 }
 
@@ -1247,6 +1271,7 @@ int state_copy(lbm_solver* s, void* host, uint64_t bytes, bool save)
         LBM_HIP(hipMemcpy(s->flags, h + kQ * plane, (size_t)s->n, hipMemcpyHostToDevice), what);
     }
     if (!save) {
+        count_written(s);
         // a saved state was stored by the same formats, hence in range
         LBM_HIP(hipMemset(s->status, 0, sizeof(uint32_t)), "hipMemset");
         s->residual_valid = 0;

@@ -115,9 +115,10 @@ struct lbm_solver {
     void* dd_alt;      // second population buffer of the out-of-place pair pass
     uint32_t* status;  // device word: nonzero after a store out of the storage range
     // the device's counter of stepped bytes (lbm_abi.cpp) at this solver's last
-    // half-step, the bytes of other solvers before that one, and its kernel
+    // half-step, the bytes of other solvers before that one, its kernel (-1: the
+    // state was written since) and whether its stores were nontemporal
     uint64_t step_mark, step_gap;
-    int last_kernel;
+    int last_kernel, streamed;
 };
 
 namespace lbm {
@@ -316,7 +317,10 @@ constexpr int kReverse = 1 << 17;     // the last cells first
 //    backwards by beta (the two gaps differ): the same, beta's range per XCD
 //    backwards; eight 82^3 FP32 322 against 344, eight 130^3 1147 against
 //    1174, four 162 x 82 x 82 FP64 494 against 521. Stepped round and round,
-//    nothing is left of them: nontemporal alpha, no reversal.
+//    nothing is left of them: nontemporal alpha, no reversal. Nor is after such
+//    an alpha (`streamed`), whatever comes between: the first alpha of eight
+//    new 128^3 streams, and their first beta backwards with the map took 680
+//    with the exchange of the faces, 620 plainly.
 //  * The 16-bit formats beyond the L2s take two neighbouring cells per thread
 //    (4-byte accesses): F16S 130^3 57.7 against 59.7 for one cell per thread,
 //    61 against 64 with others in turn; streaming, 256^3 450 against 505,
@@ -328,7 +332,8 @@ constexpr int kReverse = 1 << 17;     // the last cells first
 //    Domains with GHOST_LAYER faces store half words at their walls and ghosts,
 //    which nontemporal neighbours in the line turn into reads of the memory:
 //    always cached (250^3 462 against 519, 400^3 1890 / 2130).
-inline int step_options(const lbm_solver* s, int kernel, uint64_t near, uint64_t far)
+inline int step_options(const lbm_solver* s, int kernel, uint64_t near, uint64_t far,
+                        bool streamed)
 {
     constexpr uint64_t MB = 1ull << 20, kL2 = 40 * MB, kCache = 250 * MB;
     constexpr int NT = LBM_LAUNCH_NONTEMPORAL, XCD = LBM_LAUNCH_XCD_REMAP;
@@ -340,6 +345,8 @@ inline int step_options(const lbm_solver* s, int kernel, uint64_t near, uint64_t
         const bool by_itself = p == LBM_F32 && s->size_h[0] * s->size_h[1] % (8 * 256) == 0;
         return own <= kTinyBytes || by_itself ? 0 : XCD;
     }
+    if (streamed && own <= kCache)   // the last half-step left nothing in the cache
+        near = far = kCache;
     near += own;
     far += own;
     const bool alone = far <= own + own / 4;      // no other solvers in between

@@ -22,3 +22,29 @@ def test_first_steps_are_launched_as_later_ones(hip, precision, size):
     s.close()
     assert all(len(a) == 1 and len(b) == 1 for a, b in seen)
     assert seen[0] == seen[1] == seen[2]
+
+
+def test_first_steps_of_solvers_that_do_not_fit_together(hip):
+    """Eight solvers that fit the Infinity Cache each but not together, every state
+    written after the others' creation: alpha finds nothing of its state in the cache
+    and streams, so beta finds nothing either, also right after it."""
+    from cavityflow_cuda_amd._lib import check, lib
+    from hiprt import stream_create, stream_destroy
+    from launches import launches
+    print("[case] first steps of eight", flush=True)
+    NT, W2 = 1, 16
+    solvers = [hip.LbmSolverHIP((100, 99, 98), store_densities=False, store_velocities=False)
+               for _ in range(9)]
+    named = solvers.pop()
+    for k, options in ((0, NT | W2), (1, W2)):
+        check(lib().lbm_set_launch_options(named.handle, k, options))
+    for s in solvers:
+        s.setDensityDistributions(s.getDensityDistributions())
+    st = stream_create()
+    alpha = [launches(lambda h: s.simulationStepAlpha(stream=h), st) for s in solvers]
+    beta = [launches(lambda h: s.simulationStepBeta(stream=h), st) for s in reversed(solvers)]
+    assert alpha == [launches(lambda h: named.simulationStepAlpha(stream=h), st)] * 8
+    assert beta == [launches(lambda h: named.simulationStepBeta(stream=h), st)] * 8
+    stream_destroy(st)
+    for s in solvers + [named]:
+        s.close()
