@@ -270,7 +270,8 @@ inline uint64_t resident_bytes(const lbm_solver* s)
     return (uint64_t)s->n * (19 * s->elem_bytes + 1 + out * s->out_bytes);
 }
 
-constexpr uint64_t kTinyBytes = 2ull << 20;   // see step_options
+// Domains up to here keep plain launches (options_of_step).
+constexpr uint64_t kTinyBytes = 2ull << 20;
 
 // Internal launch options beside the LBM_LAUNCH_* ones.
 constexpr int kPairCells = 1 << 16;   // 16-bit formats: two neighbouring cells per thread
@@ -288,9 +289,12 @@ constexpr int kReverse = 1 << 17;     // the last cells first
 //    range of cells, so that its L2 still holds them, and the z neighbours of
 //    beta, from one half-step to the next: 24 x 90 x 90 FP32 13.2 against 17.7
 //    without the map, 75^3 20.4 / 23.5, 50^3 FP64 16.3 / 21.3, 75^3 F16S 17.1 /
-//    20.3. Not below 2 MB (16^3 7.1 against 6.7), and not where a slab is a
-//    multiple of 8 workgroups, which places z neighbours on one XCD by itself
-//    (62^3 FP32 15.0 against 14.0; the other formats gain there too).
+//    20.3. Slabs of a multiple of 8 workgroups, whose z neighbours lie on one XCD
+//    by themselves, gain too (FP32 3 % on average over 12 extents, 254 x 6 x 98
+//    10.8 / 14.1). FP32 and FP64 planes a multiple of 512 KiB apart share sets
+//    of the L2s, by the allocation: 62^3 FP32 12.1 or 14.3 against 13.4, with rho
+//    and u 13.5 or 15.6 / 14.1, on average over 7 such extents the same. Not
+//    below kTinyBytes (16^3 7.1 against 6.7).
 //  * All within the 256 MB Infinity Cache (one cavity stepped again and again):
 //    alpha cached and uncapped, beta with one contiguous range of cells per
 //    XCD, whose L2 then serves the lines that neighbouring workgroups share:
@@ -341,10 +345,8 @@ inline int step_options(const lbm_solver* s, int kernel, uint64_t near, uint64_t
     constexpr int LDS = LBM_LAUNCH_LDS, BIG = LBM_LAUNCH_BIG, REV = kReverse;
     const uint64_t own = resident_bytes(s);
     const int p = s->p.precision;
-    if (own <= kL2) {
-        const bool by_itself = p == LBM_F32 && s->size_h[0] * s->size_h[1] % (8 * 256) == 0;
-        return own <= kTinyBytes || by_itself ? 0 : XCD;
-    }
+    if (own <= kL2)
+        return XCD;
     if (streamed && own <= kCache)   // the last half-step left nothing in the cache
         near = far = kCache;
     near += own;
