@@ -282,7 +282,9 @@ constexpr int kReverse = 1 << 17;     // the last cells first
 // when the step starts: near and far are the lesser and the greater of the
 // bytes of other solvers stepped between this half-step and the solver's last,
 // and between that one and its predecessor. Times are us for an alpha and a
-// beta; "in turn": three solvers, one alpha and beta each.
+// beta; "in turn": three solvers, one alpha and beta each. The same launches in
+// another allocation differ by 1 to 3 %, in another process by up to 10: both
+// sides of a line were timed in one process, in several allocations.
 //  * Own bytes up to about the 8 L2s (4 MiB each): every workgroup is resident
 //    at once and no cap on the waves pays (62^3 FP32, 19 MB: 13.4 against 15.9
 //    with the streaming options). Both steps give each XCD the same contiguous
@@ -304,19 +306,22 @@ constexpr int kReverse = 1 << 17;     // the last cells first
 //    XCD map loses for FP32 and FP64; beta in 1024-thread workgroups (FP32
 //    120^3 95.0 against 98.8 in 256-thread ones, 140^3 142.6 against 147.6),
 //    FP64 at 3 waves per SIMD (110^3 140.7 against 146.9); F16S with the map
-//    (150^3 88.0 against 93.1).
+//    (150^3 88.0 against 93.1), F16C without (two 180^3 158 against 175).
 //  * The state does not fit: beta takes the cells from the last to the first
 //    (kReverse), alpha from the first. Each then starts with what the other
 //    has just left in the Infinity Cache, up to 250 MB that need not come from
 //    HBM, as long as alpha stores them there (no nontemporal alpha). 185^3 FP32
-//    321 against 351, in turn 343 against 398; 229 x 186 x 141 with outputs
-//    337 / 352, 362 / 403; 256^3 905 / 934, 921 / 966; FP64 150^3 353 / 391,
-//    381 / 433, 192^3 780 / 809, 802 / 841, 256^3 1900 / 1944. Alpha at 2 waves
-//    per SIMD, with nothing else between and below 900 MB at 4 (175^3 275
-//    against 286). FP32 beta in 1024-thread workgroups, from 1.6 GB, where the
-//    saved part is small, through LDS with nontemporal alpha (512^3 7425
-//    against 7450 without the reversal, 400^3 3581 against 3603); FP64 through
-//    LDS from 1.8 GB, with nontemporal alpha from 3 GB.
+//    320 against 351, in turn 340 against 385; 214^3 512 / 550, 529 / 570; FP64
+//    150^3 352 / 384, 377 / 414, 200^3 930 / 923, 972 / 967. Alpha at 2 waves per
+//    SIMD; FP32 up to 600 MB with nothing else between at 4 (163^3 224 against
+//    232, 185^3 320 / 330, 214^3 512 / 512; in turn 4 lose, 214^3 543 against
+//    530). Beta FP32 in 1024-thread workgroups, from 1.6 GB through LDS (235^3
+//    701 against 720, 270^3 1088 / 1087, 340^3 2217 / 2193, 420^3 4240 / 4150),
+//    FP64 through LDS from 1.8 GB (225^3 1259 against 1280, 249^3 1790 / 1767,
+//    330^3 4340 / 4130). From 3 GB alpha is nontemporal: what it leaves in the
+//    cache is little against the rest (FP64 270^3 2217 cached against 2298,
+//    290^3 2807 / 2795, 330^3 4130 / 4092; FP32 in turn 340^3 2206 / 2250, 512^3
+//    7600 / 7490).
 //  * Solvers that fit each but not together, stepped forwards by alpha and
 //    backwards by beta (the two gaps differ): the same, beta's range per XCD
 //    backwards; eight 82^3 FP32 322 against 344, eight 130^3 1147 against
@@ -329,13 +334,16 @@ constexpr int kReverse = 1 << 17;     // the last cells first
 //    (4-byte accesses): F16S 130^3 57.7 against 59.7 for one cell per thread,
 //    61 against 64 with others in turn; streaming, 256^3 450 against 505,
 //    F16C 512^3 3850 against 4060, BF16S 400^3 1769 against 1893. Within the
-//    L2s half the waves lose (62^3 13.2 against 12.4). They gain less from the
-//    reversal: with rho and u stored (200^3 F16S in turn 282 against 302,
-//    300^3 906 against 978), above 1.2 GB (512^3 3747 against 3840) and in turn
-//    up to 800 MB (220^3 309 against 316); 200^3 alone loses (244 against 238).
-//    Domains with GHOST_LAYER faces store half words at their walls and ghosts,
-//    which nontemporal neighbours in the line turn into reads of the memory:
-//    always cached (250^3 462 against 519, 400^3 1890 / 2130).
+//    L2s half the waves lose (62^3 13.2 against 12.4). Their alpha is
+//    nontemporal where nothing else comes between (F16S 200^3 211 against 225
+//    for a cached one with the reversal, 250^3 421 / 440; from 1.2 GB with the
+//    reversal, 400^3 1810 / 1840, F16C 512^3 3440 at 4 waves per SIMD and 3540
+//    at 3) and cached with the reversal in turn (200^3 235 against 245, 221^3
+//    309 / 340, 270^3 557 / 560) and with rho and u stored below 1.2 GB (221^3
+//    356 / 385, 270^3 661 / 724). Domains with GHOST_LAYER faces store half words
+//    at their walls and ghosts, which nontemporal neighbours in the line turn
+//    into reads of the memory: always cached (250^3 462 against 519, 400^3 1890
+//    / 2130).
 inline int step_options(const lbm_solver* s, int kernel, uint64_t near, uint64_t far,
                         bool streamed)
 {
@@ -355,43 +363,32 @@ inline int step_options(const lbm_solver* s, int kernel, uint64_t near, uint64_t
     const bool to_and_fro = far >= near + own / 2;
     auto opts = [&](int alpha, int beta) { return kernel == 0 ? alpha : beta; };
     if (p != LBM_F32 && p != LBM_F64) {
-        const bool wide_codes = p == LBM_F16C;    // more integer work per cell
+        const bool open = !is_closed(s), large = own > 1200 * MB;
         const bool outputs = s->p.store_densities || s->p.store_velocities;
         int o;
         if (near <= kCache)
-            o = far <= 300 * MB ? opts(0, XCD | W4) : wide_codes ? W4 : opts(W4, XCD | W3);
+            o = far <= 300 * MB ? opts(0, XCD | W4) : p == LBM_F16C ? W4 : opts(W4, XCD | W3);
         else if (own <= kCache)
-            o = opts(NT | W3, XCD | (wide_codes ? W4 : W3));
-        else if (own > 1200 * MB || (outputs && own > 800 * MB))
-            o = wide_codes ? opts(NT | W4, W4 | REV) : opts(NT | W3, W3 | REV);
-        else if (own > 800 * MB)
-            o = opts(NT | W3, wide_codes ? W4 : W3);
-        else if (outputs)
-            o = opts(W3, W3 | REV);
-        else if (alone || own <= 300 * MB)
-            o = own <= 500 * MB ? opts(NT | W4, W4) : opts(NT | W3, wide_codes ? W4 : W3);
-        else
+            o = opts(open ? W3 : NT | W3, XCD | W4);
+        else if (open || (!large && (outputs || !alone)))
             o = opts(W3, W4 | REV);
-        return kPairCells | (is_closed(s) ? o : o & ~NT);
+        else if (!large)
+            o = opts(NT | W4, W4);
+        else   // F16C has more integer work per cell
+            o = p == LBM_F16C ? opts(NT | W4, W4 | REV) : opts(NT | W3, W3 | REV);
+        return kPairCells | o;
     }
     if (near <= kCache && far <= 300 * MB)
         return opts(0, XCD | (p == LBM_F32 ? W2 : W3));
     if (near <= kCache)
         return p == LBM_F32 ? opts(W3, BIG | W4) : opts(W2, W3);
-    if (own <= kCache) {
-        if (!to_and_fro)
-            return opts(NT | W2, W2);
-        const uint64_t all = (near + far) / 2;
-        return opts(p == LBM_F32 && all <= 600 * MB ? W3 : W2, XCD | W3 | REV);
-    }
-    if (p == LBM_F32) {
-        if (own >= 1600 * MB)
-            return opts(NT | W2, LDS | W4 | REV);
-        return opts(alone && own <= 900 * MB ? W4 : own <= 300 * MB ? W3 : W2, BIG | W4 | REV);
-    }
-    if (own < 1800 * MB)
-        return opts(W2, (own <= 800 * MB ? W3 : W2) | REV);
-    return opts((own < 3000 * MB ? 0 : NT) | W2, LDS | W2 | REV);
+    if (own <= kCache)
+        return to_and_fro ? opts(W2, XCD | W3 | REV) : opts(NT | W2, W2);
+    const int huge = own < 3000 * MB ? 0 : NT;
+    if (p == LBM_F32)
+        return own >= 1600 * MB ? opts(huge | W2, LDS | W4 | REV)
+                                : opts(alone && own <= 600 * MB ? W4 : W2, BIG | W4 | REV);
+    return opts(huge | W2, (own < 1800 * MB ? 0 : LDS) | W2 | REV);
 }
 
 // ||u - u_prev|| / ||u|| from the two FP64 sums; a non-finite state gives NaN

@@ -1,4 +1,6 @@
-"""The launch options that whole-domain steps choose, compiled for the host."""
+"""The launch options that whole-domain steps choose, compiled for the host: every
+line of the choice at sizes on both of its sides, and that the sizes of the GPU tests
+of the choice lie in the part that each is there for."""
 import os
 import shutil
 import subprocess
@@ -23,6 +25,51 @@ ROWS = [
     ("f32", (37, 33, 31), 0, WALL, 0, 0, X, X), ("f32", (62, 62, 62), 0, WALL, 0, 0, X, X),
     ("f32", (62, 62, 62), 1, WALL, 500, 500, X, X), ("f64", (59, 59, 59), 0, WALL, 0, 0, X, X),
     ("f16s", (75, 74, 73), 1, WALL, 0, 0, X, X), ("f16c", (91, 87, 83), 0, GHOST, 0, 0, X, X),
+    # all within the Infinity Cache
+    ("f32", (86, 83, 81), 0, WALL, 0, 0, 0, X | W2), ("f64", (70, 69, 67), 0, WALL, 0, 0, 0, X | W3),
+    ("f16s", (107, 103, 101), 0, WALL, 0, 0, P, P | X | W4),
+    ("f16c", (107, 103, 101), 0, WALL, 0, 0, P, P | X | W4),
+    ("bf16s", (107, 103, 101), 0, WALL, 0, 0, P, P | X | W4),
+    # only the state itself
+    ("f32", (86, 83, 81), 0, WALL, 0, 348, W3, BIG | W4),
+    ("f64", (70, 69, 67), 0, WALL, 0, 348, W2, W3),
+    ("f16s", (107, 103, 101), 0, WALL, 0, 348, P | W4, P | X | W3),
+    ("f16c", (107, 103, 101), 0, WALL, 0, 348, P | W4, P | W4),
+    # fits, but not with the others: round and round, to and fro
+    ("f32", (86, 83, 81), 0, WALL, 348, 348, NT | W2, W2),
+    ("f32", (86, 83, 81), 0, WALL, 220, 348, W2, X | W3 | REV),
+    ("f64", (70, 69, 67), 0, WALL, 220, 500, W2, X | W3 | REV),
+    ("f16s", (107, 103, 101), 0, WALL, 348, 348, P | NT | W3, P | X | W4),
+    ("f16s", (107, 103, 101), 0, GHOST, 348, 348, P | W3, P | X | W4),
+    # nontemporal stores left nothing in the cache, whatever came between
+    ("f32", (86, 83, 81), 0, WALL, 0, 348, NT | W2, W2, 1),
+    ("f64", (70, 69, 67), 0, WALL, 0, 0, NT | W2, W2, 1),
+    ("f16s", (107, 103, 101), 0, WALL, 0, 0, P | NT | W3, P | X | W4, 1),
+    ("f16s", (190, 187, 193), 0, WALL, 0, 0, P | NT | W4, P | W4, 1),
+    # larger than the cache
+    ("f32", (151, 149, 150), 0, WALL, 0, 0, W4, BIG | W4 | REV),
+    ("f32", (229, 186, 141), 1, WALL, 0, 0, W4, BIG | W4 | REV),
+    ("f32", (229, 186, 141), 1, WALL, 0, 348, W2, BIG | W4 | REV),
+    ("f32", (217, 217, 217), 0, WALL, 0, 0, W2, BIG | W4 | REV),
+    ("f32", (275, 275, 275), 0, WALL, 0, 0, W2, BIG | W4 | REV),
+    ("f32", (281, 280, 279), 0, WALL, 0, 0, W2, LDS | W4 | REV),
+    ("f32", (350, 345, 345), 0, WALL, 0, 0, NT | W2, LDS | W4 | REV),
+    ("f64", (150, 147, 139), 0, WALL, 0, 0, W2, W2 | REV),
+    ("f64", (227, 226, 225), 0, WALL, 0, 0, W2, W2 | REV),
+    ("f64", (233, 232, 231), 0, WALL, 0, 0, W2, LDS | W2 | REV),
+    ("f64", (280, 271, 275), 0, WALL, 0, 0, NT | W2, LDS | W2 | REV),
+    ("f16s", (190, 187, 193), 0, WALL, 0, 0, P | NT | W4, P | W4),
+    ("f16c", (221, 219, 220), 0, WALL, 0, 0, P | NT | W4, P | W4),
+    ("f16s", (190, 187, 193), 0, WALL, 0, 348, P | W3, P | W4 | REV),
+    ("f16s", (205, 203, 199), 1, WALL, 0, 0, P | W3, P | W4 | REV),
+    ("bf16s", (241, 260, 277), 1, WALL, 0, 0, P | W3, P | W4 | REV),
+    ("bf16s", (300, 290, 277), 1, WALL, 0, 0, P | NT | W3, P | W3 | REV),
+    ("f16s", (321, 319, 320), 0, WALL, 0, 0, P | NT | W3, P | W3 | REV),
+    ("f16c", (321, 319, 320), 0, WALL, 0, 0, P | NT | W4, P | W4 | REV),
+    # exchanged faces: never nontemporal
+    ("f16s", (190, 187, 193), 0, GHOST, 0, 0, P | W3, P | W4 | REV),
+    ("f16c", (321, 319, 320), 0, GHOST, 0, 0, P | W3, P | W4 | REV),
+    ("f32", (281, 280, 279), 0, GHOST, 0, 0, W2, LDS | W4 | REV),
 ]
 
 
