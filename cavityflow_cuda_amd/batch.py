@@ -113,7 +113,9 @@ class CavityBatch:
         the current ones (initially the precision's defaults); pairs=1 runs
         each alpha + beta pair as one out-of-place pass (then run() needs
         multiples of 4 steps); group_mb > 0 runs the members in groups of at
-        most that many MiB of populations, one group after the other."""
+        most that many MiB of populations, one group after the other. What
+        tuning() reports before any other was set stands for a choice by size
+        (include/lbm_abi.h), also when it is set again unchanged."""
         if options is None:
             options = self.tuning()["options"]
         t = _lib.lbm_batch_tuning(block, cells_per_thread, waves_per_cu,

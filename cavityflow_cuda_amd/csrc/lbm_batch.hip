@@ -23,6 +23,7 @@
 #include "lbm_abi.h"
 #include "lbm_cell.hpp"
 #include "lbm_pair.hpp"
+#include "lbm_tuner.hpp"
 
 namespace lbm {
 
@@ -182,7 +183,7 @@ struct lbm_batch {
     };
     std::vector<Group> groups;
     uint64_t bytes = 0;        // of all members' populations
-    bool tuned = false;        // the caller set (or autotuned) the tuning
+    bool tuned = false;        // a tuning other than start_tuning is set
     int cpt = 1;               // cells per thread of the launches
     ResidualMember* res_mem = nullptr;   // members' residual inputs
     double* res_part = nullptr;          // members * kReduceBlocks * 5 partial sums
@@ -258,10 +259,6 @@ int upload_tiles(lbm_batch* b, uint32_t tile_cells, std::vector<MemberDesc>& des
     return LBM_OK;
 }
 
-// candidates besides the starting tuning that the autotuner's final round
-// times again over longer runs
-constexpr size_t kFinalists = 4;
-
 constexpr int kBatchOptions =
     LBM_LAUNCH_NONTEMPORAL | LBM_LAUNCH_XCD_REMAP | LBM_LAUNCH_WAVES4 | LBM_LAUNCH_WAVES3 |
     LBM_LAUNCH_WAVES2;
@@ -275,6 +272,18 @@ static int batch_start_options(int precision, int kernel)
     if (precision == LBM_F32 || precision == LBM_F64)
         return default_launch(precision, kernel, true, false) & kBatchOptions;
     return kernel == 0 ? LBM_LAUNCH_NONTEMPORAL : 0;
+}
+
+// The tuning a batch is created with. It stands for the choice below: a batch
+// that has it, reported and set back or never set, is not tuned.
+static lbm_batch_tuning start_tuning(int precision)
+{
+    lbm_batch_tuning t{};
+    t.block = 256;
+    t.cells_per_thread = 1;
+    for (int kernel = 0; kernel < 2; kernel++)
+        t.options[kernel] = batch_start_options(precision, kernel);
+    return t;
 }
 
 // A batch whose tuning the caller has not set runs its members in groups that
@@ -336,13 +345,6 @@ size_t waves_lds(int opts, int block)
         return 0;
     const int per_cu = std::max(1, waves * 4 / (block / 64));   // workgroups per CU
     return (size_t)(160 * 1024) / (size_t)(per_cu + 1) + 1024;
-}
-
-bool same_tuning(const lbm_batch_tuning& a, const lbm_batch_tuning& b)
-{
-    return a.block == b.block && a.cells_per_thread == b.cells_per_thread &&
-           a.waves_per_cu == b.waves_per_cu && a.options[0] == b.options[0] &&
-           a.options[1] == b.options[1] && a.pairs == b.pairs && a.group_mb == b.group_mb;
 }
 
 bool valid_tuning(const lbm_batch_tuning& t)
@@ -470,6 +472,7 @@ int apply_tuning(lbm_batch* b, const lbm_batch_tuning& t)
         free_alt(b);           // no pair pass: no second population buffers
     }
     b->tuning = t;
+    b->tuned = !same_tuning(t, start_tuning(b->precision));
     b->bytes = 0;
     for (const lbm_solver* s : b->members)
         b->bytes += (uint64_t)kQ * s->stride * s->elem_bytes;
@@ -711,17 +714,7 @@ int lbm_batch_create(lbm_solver* const* members, int count, lbm_batch** out)
         d.rest_rho = gravity_product(d.g0, d.g1, d.g2);
         d.status = s->status;
     }
-    lbm_batch_tuning t;
-    t.block = 256;
-    t.cells_per_thread = 1;
-    t.waves_per_cu = 0;
-    // the batch kernels take their shape from the tuning (block,
-    // cells_per_thread)
-    t.options[0] = batch_start_options(b->precision, 0);
-    t.options[1] = batch_start_options(b->precision, 1);
-    t.pairs = 0;
-    t.group_mb = 0;
-    if ((rc = apply_tuning(b, t))) {
+    if ((rc = apply_tuning(b, start_tuning(prec)))) {
         lbm_batch_destroy(b);
         return rc;
     }
@@ -757,11 +750,7 @@ int lbm_batch_set_tuning(lbm_batch* b, const lbm_batch_tuning* t)
     int rc = set_dev(b->device);
     if (rc)
         return rc;
-    const bool before = b->tuned;
-    b->tuned = true;
-    if ((rc = apply_tuning(b, *t)))
-        b->tuned = before;
-    return rc;
+    return apply_tuning(b, *t);
 }
 
 int lbm_batch_get_tuning(const lbm_batch* b, lbm_batch_tuning* t)
@@ -860,12 +849,8 @@ int lbm_batch_autotune(lbm_batch* b, int trial_steps, hipStream_t stream,
     int rc = set_dev(b->device);
     if (rc)
         return rc;
-    // Trials time whole steps (alpha then beta), since each phase's speed
-    // depends on what the other leaves in the caches: first the workgroup
-    // shape with the current launch options, then alpha's options with beta's
-    // fixed, then beta's with the chosen alpha, then the pair pass. The
-    // members' state advances by whole steps during the trials (an even
-    // number of pair passes), exactly as in a run.
+    // the members' state advances by whole steps during the trials (an even
+    // number of pair passes), exactly as in a run
     // the two timing events live until every return path of the tuner
     struct Events {
         hipEvent_t e[2] = {nullptr, nullptr};
@@ -899,138 +884,21 @@ int lbm_batch_autotune(lbm_batch* b, int trial_steps, hipStream_t stream,
         *per_step = ms / (float)whole;
         return LBM_OK;
     };
-    b->tuned = true;   // every trial runs the tuning it names
-    lbm_batch_tuning best = b->tuning;
-    best.pairs = 0;
-    float best_step = std::numeric_limits<float>::infinity();
-    std::vector<std::pair<float, lbm_batch_tuning>> timed;   // every trial, for the final round
-    auto consider = [&](const lbm_batch_tuning& c) -> int {
-        float t = 0.f;
-        const int r = step_time(c, trial_steps, &t);
-        if (r)
-            return r;
-        timed.push_back({t, c});
-        if (t < best_step) {
-            best_step = t;
-            best = c;
-        }
-        return LBM_OK;
-    };
-    const lbm_batch_tuning start = best;
-    // 1024-thread workgroups: not for FP64 (apply_tuning), and at most two are
-    // resident per CU
-    const int max_block = b->precision == LBM_F64 ? 512 : 1024;
-    for (int blk : {256, 512, 1024})
-        for (int cpt : {1, 2, 4})
-            for (int wpc : {0, 1, 2, 3, 4, 8, 16}) {
-                if (blk > max_block || (blk == 1024 && wpc > 2))
-                    continue;
-                lbm_batch_tuning cand = start;
-                cand.block = blk;
-                cand.cells_per_thread = cpt;
-                cand.waves_per_cu = wpc;
-                if ((rc = consider(cand)))
-                    return rc;
-            }
-    for (int ph = 0; ph < 2; ph++) {
-        const lbm_batch_tuning shape = best;
-        for (int opt : {0, 1, 2, 3, 4, 5, 6, 8, 9, 16, 17}) {
-            lbm_batch_tuning cand = shape;
-            cand.options[ph] = opt;
-            if ((rc = consider(cand)))
-                return rc;
-        }
-    }
-    // member groups small enough for the last-level cache to keep their state
-    // between consecutive steps
-    {
-        const lbm_batch_tuning ungrouped = best;
-        for (int mb : {32, 64, 128, 192, 256, 384}) {
-            lbm_batch_tuning cand = ungrouped;
-            cand.group_mb = mb;
-            if ((rc = consider(cand)))
-                return rc;
-        }
-        // what a batch without a set tuning launches
-        lbm_batch_tuning cand = start;
-        cand.block = 256;
-        cand.cells_per_thread = pairs_pay(b) ? 2 : 1;
-        cand.waves_per_cu = 0;
-        cand.group_mb = (int)(kCacheGroup >> 20);
-        for (int ph = 0; ph < 2; ph++)
-            cand.options[ph] = cached_options(b, ph);
-        if ((rc = consider(cand)))
-            return rc;
-    }
-    // with the state of a group in the cache the best workgroup shape can
-    // differ from the streaming one: the shapes once more, grouped
-    if (best.group_mb > 0) {
-        const lbm_batch_tuning grouped = best;
-        for (int blk : {256, 512, 1024})
-            for (int cpt : {1, 2, 4}) {
-                if (blk > max_block || (blk == 1024 && grouped.waves_per_cu > 2))
-                    continue;
-                lbm_batch_tuning cand = grouped;
-                cand.block = blk;
-                cand.cells_per_thread = cpt;
-                if ((rc = consider(cand)))
-                    return rc;
-            }
-    }
-    // the pair pass, when the members allow it
-    bool eligible = true;
-    for (int shape = 1; shape <= kPairShapes && eligible; shape++)
-        for (int opt = 0; opt < 4; opt++) {
-            lbm_batch_tuning cand = best;
-            cand.pairs = shape;
-            cand.group_mb = 0;
-            cand.options[0] = opt;
-            if (apply_tuning(b, cand) != LBM_OK) {
-                eligible = false;   // not eligible: keep the in-place launches
-                break;
-            }
-            float t = 0.f;
-            if ((rc = step_time(cand, trial_steps, &t)))
-                return rc;
-            timed.push_back({t, cand});
-            if (t < best_step) {
-                best_step = t;
-                best = cand;
-            }
-        }
-    // Short trials are noisy, and the more candidates, the likelier a lucky
-    // trial wins: the few fastest distinct candidates and the starting tuning
-    // run again over longer runs, interleaved, and the least total time wins
-    // (the starting tuning on a tie).
-    std::stable_sort(timed.begin(), timed.end(),
-                     [](const auto& x, const auto& y) { return x.first < y.first; });
-    std::vector<lbm_batch_tuning> finalists{start};
-    for (const auto& tc : timed) {
-        if (finalists.size() > kFinalists)
-            break;
-        bool seen = false;
-        for (const lbm_batch_tuning& f : finalists)
-            seen = seen || same_tuning(f, tc.second);
-        if (!seen)
-            finalists.push_back(tc.second);
-    }
-    if (finalists.size() > 1) {
-        const int long_steps = 4 * trial_steps;
-        std::vector<float> total(finalists.size(), 0.f);
-        for (int rep = 0; rep < 2; rep++)
-            for (size_t i = 0; i < finalists.size(); i++) {
-                float t = 0.f;
-                if ((rc = step_time(finalists[i], long_steps, &t)))
-                    return rc;
-                total[i] += t;
-            }
-        size_t win = 0;
-        for (size_t i = 1; i < finalists.size(); i++)
-            if (total[i] < total[win])
-                win = i;
-        best = finalists[win];
-    }
-    if ((rc = apply_tuning(b, best)))
+    lbm_batch_tuning start = b->tuning;
+    start.pairs = 0;
+    // the launches of a batch without a set tuning for members that stay in the
+    // cache, with their shape and their two options for all groups alike
+    lbm_batch_tuning cached = start_tuning(b->precision);
+    cached.cells_per_thread = pairs_pay(b) ? 2 : 1;
+    cached.group_mb = (int)(kCacheGroup >> 20);
+    for (int ph = 0; ph < 2; ph++)
+        cached.options[ph] = cached_options(b, ph);
+    lbm_batch_tuning best;
+    const int max_block = b->precision == LBM_F64 ? 512 : 1024;   // apply_tuning
+    auto allowed = [&](const lbm_batch_tuning& c) { return apply_tuning(b, c) == LBM_OK; };
+    if ((rc = search_tuning(start, start_tuning(b->precision), cached, max_block, kPairShapes,
+                            trial_steps, step_time, allowed, &best)) ||
+        (rc = apply_tuning(b, best)))
         return rc;
     if (chosen)
         *chosen = best;

@@ -475,10 +475,14 @@ typedef struct lbm_batch_tuning {
                               Not with pairs. */
 } lbm_batch_tuning;
 
-/* A batch whose tuning was neither set nor autotuned runs 256-thread tiles as
- * lbm_batch_get_tuning reports them, but in groups of at most 224 MiB, with
- * launch options chosen by whether a group's state stays in the last-level
- * cache between its half-steps. */
+/* The tuning a batch is created with stands for a choice by size: groups of at
+ * most 224 MiB, 256-thread tiles of one cell per thread (16-bit formats beyond
+ * the L2s: two neighbouring ones), and for each group launch options by whether
+ * its state stays in the last-level cache between its half-steps.
+ * lbm_batch_get_tuning reports the created tuning's own fields, one launch over
+ * all members; set back with every field unchanged it stands for the choice
+ * again. A tuning that differs in any field is launched as its fields say: to
+ * change one field of the choice, set group_mb too. */
 
 int lbm_batch_create(lbm_solver* const* members, int count, lbm_batch** out);
 int lbm_batch_destroy(lbm_batch* batch);
@@ -500,9 +504,10 @@ int lbm_batch_launch(lbm_batch* batch, int first_phase, int half_steps, hipStrea
  * options, member groups with the shapes again under the chosen group, and
  * the pair pass when the members allow it) as runs of trial_steps whole steps
  * (lbm_batch_run: graph-captured on a non-NULL stream, direct launches on the
- * NULL stream); the four fastest distinct candidates and the starting tuning
- * then run again over runs four times as long, interleaved, and the least
- * total time wins (the starting tuning on a tie).
+ * NULL stream); the four fastest distinct candidates, the tuning the batch has
+ * and the one it was created with (above) then run again over runs four times
+ * as long, interleaved, and the least total time wins (the tuning it has on a
+ * tie).
  * The trials are real steps: the members advance; reset them afterwards
  * (lbm_reset) when their state matters. Synchronous. */
 int lbm_batch_autotune(lbm_batch* batch, int trial_steps, hipStream_t stream,
