@@ -45,14 +45,16 @@ bool take_ring()
     return true;
 }
 
-bool is_pinned(const void* p)
+// Memory the runtime does not know. What it knows, pinned, managed or the
+// device's, it copies itself: the workers' memcpy is for host pages alone.
+bool is_pageable(const void* p)
 {
     hipPointerAttribute_t a;
     if (hipPointerGetAttributes(&a, p) != hipSuccess) {
-        (void)hipGetLastError();   // pageable memory the runtime does not know
-        return false;
+        (void)hipGetLastError();
+        return true;
     }
-    return a.type == hipMemoryTypeHost;
+    return a.type == hipMemoryTypeUnregistered;
 }
 
 // Workers that copy their share of chunk 0, 1, ... between the ring and the
@@ -219,7 +221,7 @@ hipError_t through_ring(const std::vector<Segment>& chunks, bool to_host, hipStr
 
 bool ring_pays(const void* host, size_t bytes, size_t segments)
 {
-    return bytes >= (segments > 1 ? kLeastOfMany : kLeast) && !is_pinned(host);
+    return bytes >= (segments > 1 ? kLeastOfMany : kLeast) && is_pageable(host);
 }
 
 hipError_t transfer(const Segment* segments, size_t count, bool to_host, hipStream_t st)
