@@ -455,8 +455,9 @@ int check_params(const lbm_params& p, const char* who, int64_t* cells)
 // of 2 MiB apart (64^3 FP64, 128^3, 256^3, 512^3 cells with the walls) would put
 // a cell's 19 values into the same sets of the caches and channels of the
 // memory; those lie 9 * 256 elements further apart. us for an alpha and a beta: FP32
-// 254^3 977 -> 874, 510^3 6980-7160 -> 6830-6900, three 126^3 in turn 131 -> 116;
-// FP64 126^3 235 -> 210; F16S 126^3 57.2 -> 54.2, 510^3 3740 -> 3460-3640.
+// 254^3 977 -> 874, three 126^3 in turn 131 -> 116; FP64 126^3 235 -> 210; F16S
+// 126^3 57.2 -> 54.2. At 510^3 the gain (FP32 6980 -> 6870, F16S 3740 -> 3550) is
+// within what the place of the allocation changes by itself.
 static int64_t plane_stride(int64_t n, int elem_bytes)
 {
     const int64_t stride = (n + 255) / 256 * 256;

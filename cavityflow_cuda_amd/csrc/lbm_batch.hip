@@ -455,8 +455,8 @@ int prepare_pairs(lbm_batch* b, int pairs)
 int apply_tuning(lbm_batch* b, const lbm_batch_tuning& t)
 {
     if (t.block == 1024 && b->precision == LBM_F64) {
-        // a limit from when the FP64 kernels needed more than the 128 VGPRs of
-        // such a workgroup's threads (87 and 71 now)
+        // such a workgroup's threads have 128 VGPRs each, which the FP64 kernels
+        // once exceeded (90 and 67 now); kept, as callers rely on the error
         set_error("batch tuning: FP64 members take workgroups of 256 or 512 threads");
         return LBM_ERR_UNSUPPORTED;
     }

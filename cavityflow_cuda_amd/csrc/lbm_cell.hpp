@@ -626,8 +626,8 @@ struct HalfOutputs {
 // (store_walls): without them no row's first and last lines are whole, and the
 // memory then reads what it writes (512^3 F16S 3925 us for an alpha and a beta
 // against 3740, 250^3 462 against 421; with nontemporal stores 4360 and 519).
-// Bound by memory: F16S 512^3 moves its 20.8 GB of an alpha and a beta in
-// 3690 us, 5.6 TB/s (one cell per thread 4050 us).
+// Bound by memory: F16S 512^3 moves its 20.8 GB of an alpha and a beta in 3740 to
+// 3880 us by the allocation, 5.4 to 5.6 TB/s (one cell per thread 4050 to 4180).
 template <class S>
 struct AccHalf {
     uint32_t* word;   // [19], registers

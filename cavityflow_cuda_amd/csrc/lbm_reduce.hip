@@ -454,9 +454,10 @@ hipError_t launch_residual_members(int precision, const ResidualMember* mem, int
 // holds its own copy until the process ends. In host code `scratch` names a
 // host-side stand-in, not a device address, so it is never passed to a kernel
 // or a copy: each device's address comes from hipGetSymbolAddress, looked up
-// once per device with that device current (noalloc_scratch). Every block
-// overwrites its whole slice, so nothing has to start at zero; two calls that
-// overlap on one GPU share the array and race.
+// once per device with that device current (noalloc_scratch). Nothing has to
+// start at zero: the final sum reads the slots of the reduce_blocks(cells)
+// blocks that have cells, and those have written theirs. Two calls that overlap
+// on one GPU share the array and race.
 static __device__ __align__(256) double scratch[LBM_NOALLOC_MAX_BOXES * kReduceBlocks * kRedVals];
 
 static std::mutex g_scratch_mutex;
